@@ -74,16 +74,16 @@ size_t bfk_ortho_units(int rows, int n);
 int bfk_ortho(const BfkOrthoJob *dJobs, const int32_t *dOrder, int numGroups, const int64_t *groupStart,
               const size_t *groupBytes, const BfkOrthoItem *dItems, double *dArena, const double *dRin,
               double *dRout);
-int bfk_apply(const BfkSeg *dSegs, const int64_t *stageSeg, int numStages, const BfkTerm *dTerms,
+int bfk_apply(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int numStages, const BfkTerm *dTerms,
               const double *dArena, const double *dX, double *dPing, double *dPong, double *dY, int nrhs,
               const int32_t *stageCfg);
-int bfk_apply_f32(const BfkSeg *dSegs, const int64_t *stageSeg, int numStages, const BfkTerm *dTerms,
+int bfk_apply_f32(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int numStages, const BfkTerm *dTerms,
                   const float *dArenaHi, const float *dArenaLo, const float *dX, float *dPing, float *dPong,
                   float *dY, int nrhs, const int32_t *stageCfg);
-int bfk_apply_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, int s, const BfkTerm *dTerms,
+int bfk_apply_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int s, const BfkTerm *dTerms,
                        const double *dArena, const double *dX, double *dPing, double *dPong, double *dY, int nrhs,
                        int cfg, int reps, double *ms);
-int bfk_apply_f32_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, int s, const BfkTerm *dTerms,
+int bfk_apply_f32_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int s, const BfkTerm *dTerms,
                            const float *dArenaHi, const float *dArenaLo, const float *dX, float *dPing, float *dPong,
                            float *dY, int nrhs, int cfg, int reps, double *ms);
 int bfk_graph_begin(void);
@@ -179,6 +179,7 @@ typedef struct BfMatHipButterfly {
   BfSegVec segs;
   BfTermVec terms;
   BfI64Vec stageSeg;
+  BfkStageShape *stageShape; /* one per stage */
   int numStages;
   int64_t bufRows[3];  /* rows of ping, pong (per right-hand side) */
   double applyFactorBytes;
@@ -221,6 +222,8 @@ int bfPlanButterfly(BfMatHipButterfly *F, BfQuadtree const *src, BfQuadtree cons
                     const size_t *nls, const int32_t *const *lt, const size_t *nlt, int D);
 /* apply plan (fac.c) */
 int bfApplyPlanBuild(BfMatHipButterfly *F);
+/* the shapes of an apply plan's stages; NULL without memory */
+BfkStageShape *bfStageShapes(const BfkSeg *segs, const int64_t *stageSeg, int numStages, const BfkTerm *terms);
 /* apply plan and uploads for a plan + arena already in place (fac.c) */
 int bfMatHipButterflyFinish(BfMatHipButterfly *F);
 

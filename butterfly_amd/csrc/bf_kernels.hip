@@ -10,11 +10,12 @@
  *              the augmented [Z_equiv | Z_orig], then
  *              X = Z_equiv^+ Z_orig with the reference's truncation
  *              (helm2.c:321-365, mat_dense_complex.c:1768-1849)
- *   k_apply1   one stage of the apply for one right-hand side: every
- *              output row segment sums its column-major blocks times the
- *              input (mat_product.c:211-245, mat_block_coo.c:382-425,
- *              mat_block_diag.c:372-407, mat_block_dense.c:512-572)
- *   k_applyN   the same for many right-hand sides (one lane per column)
+ *   k_applyN_mfma  one stage of the apply for many right-hand sides on the
+ *              matrix cores: every output row segment sums its column-major
+ *              blocks times the input (mat_product.c:211-245,
+ *              mat_block_coo.c:382-425, mat_block_diag.c:372-407,
+ *              mat_block_dense.c:512-572); one and a few right-hand sides
+ *              are in bf_apply_few.hip
  *
  * One wave64 per job / segment; all jobs of a level or stage go into one
  * launch.  Everything here is FP64 unless the name says f32.
@@ -25,6 +26,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include "bf_apply.h"
 #include "bf_h0.h"
 #include "bf_plan.h"
 
@@ -1709,51 +1711,20 @@ __global__ __launch_bounds__(64) void k_ortho(const BfkOrthoJob *__restrict__ jo
 
 /* ---------------------------------------------------------------- apply */
 
-struct BfkBufs {
-  const double2 *in[4];
-  double2 *out[4];
-};
-
-struct BfkBufsF {
-  const float2 *in[4];
-  float2 *out[4];
-};
-
-__device__ __forceinline__ float2 cfmaf(float2 a, float2 b, float2 c) {
-  return make_float2(fmaf(a.x, b.x, fmaf(-a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, c.y)));
-}
-__device__ __forceinline__ double2 cfmaT(double2 a, double2 b, double2 c) { return cfma(a, b, c); }
-__device__ __forceinline__ float2 cfmaT(float2 a, float2 b, float2 c) { return cfmaf(a, b, c); }
 template <typename V> __device__ __forceinline__ V czero();
 template <> __device__ __forceinline__ double2 czero<double2>() { return make_double2(0, 0); }
 template <> __device__ __forceinline__ float2 czero<float2>() { return make_float2(0, 0); }
-template <typename V> __device__ __forceinline__ V cadd(V a, V b) {
-  a.x += b.x;
-  a.y += b.y;
-  return a;
-}
 
-template <typename V> struct BufsOf;
-template <> struct BufsOf<double2> { typedef BfkBufs T; };
-template <> struct BufsOf<float2> { typedef BfkBufsF T; };
-
-/* compensated (Kahan) accumulation: s + (-c) carries the running sum to
- * about one rounding of the final value however long the chain */
 /* add an FP32 accumulator tile into an FP64 running sum and clear it */
 typedef double mf_d4 __attribute__((ext_vector_type(4)));
 template <class A> __device__ __forceinline__ void fold64(mf_d4 &s, A &p) {
   s += __builtin_convertvector(p, mf_d4);
   p = A{};
 }
-__device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
-  return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
-}
 
-/* Launch shape of the 1-RHS apply: waves (segments) per block and the lane
- * map (0 = rows = segment height, 1 = the next power of two); set by
- * bfk_set_apply_config. */
+/* segments (waves) per block of the one- and few-RHS apply; set by
+ * bfk_set_apply_config */
 static int g_applyWaves = 1;
-static int g_applyUnroll = 0;
 /* the MFMA apply's shape: right-hand-side tiles of 16 per wave | 16 for
  * two row tiles per wave (0 = the vector-unit kernel, -1 = the defaults
  * below, the shapes the tuner picks at N = 2^20) */
@@ -1773,211 +1744,6 @@ static int g_comp32 = 2;
  * (mask + 1) 4-column steps */
 static int g_foldMask = 0;
 __constant__ int g_foldMaskDev = 0;
-
-/* One stage of the apply for one right-hand side.  Each wave of the block
- * owns one output row segment: its lanes split into R rows x G = 64/R
- * column groups (R = the segment height, at most 64; UNROLL selects the
- * next power of two instead); a lane walks its columns of every term
- * (column-major blocks, so the R lanes of a group read R consecutive
- * entries), then the G partial sums meet through lane reads and the row is
- * written once.  The walk is software-pipelined: a lane's columns go in
- * batches of two, a batch never spanning two terms, and the loads of the
- * next batch are issued before the products of the current one, so a wave
- * has two batches of loads in flight across term boundaries.  Loads never
- * branch: columns past a term's width read its last column and are masked
- * out by a select.  With LO the factors are an FP32 pair hi + lo.  With
- * COMP (FP32 only) every lane sums its products in FP64 (two chains) and
- * the lanes of a row meet in FP64, so the rounding of a stage no longer
- * grows with the length of its rows; with LO and COMP the pair is summed
- * and multiplied in FP64. */
-template <typename V, bool LO, bool UNROLL, bool COMP = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_apply1(const BfkSeg *__restrict__ segs, int64_t numSegs,
-                                                const BfkTerm *__restrict__ terms, const V *__restrict__ hi,
-                                                const V *__restrict__ lo, typename BufsOf<V>::T bufs) {
-  const int lane = threadIdx.x & 63;
-  /* the wave's segment index as a wave-uniform value, so the segment and
-   * term descriptors come through scalar loads */
-  const int64_t si = (int64_t)blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (si >= numSegs) return; /* whole wave; no block barrier below */
-  const BfkSeg S = segs[si];
-  const int m = S.m;
-  /* lane map: Rm rows x Gm column groups; the tight map (rows = segment
-   * height) keeps 51 of 64 lanes busy on a 17-row segment where the
-   * power-of-two map keeps 34 (4.4% faster at N = 2^20) */
-  int Rm;
-  if (UNROLL && !COMP) {
-    Rm = 64;
-    while (Rm > 1 && (Rm >> 1) >= m) Rm >>= 1;
-  } else {
-    Rm = m < 64 ? m : 64;
-  }
-  const int Gm = 64 / Rm, rl = lane % Rm, gl = lane / Rm;
-  /* columns per lane per batch: two FP64 batches of two fit seven waves
-   * per SIMD without spills; the compensated FP32 form measured 9.2 ms
-   * with two against 10.5 ms with three at N = 2^20 */
-  constexpr int APPLY1_BATCH = 2;
-  V *y = bufs.out[S.ybuf] + S.yOff;
-  /* batches over the block terms: ceil(n / (APPLY1_BATCH Gm)) per term */
-  const int span = APPLY1_BATCH * Gm;
-  int batches = 0;
-  for (int t = S.t0; t < S.t1; ++t) {
-    const BfkTerm T = terms[t];
-    if (T.aOff >= 0) batches += (T.n + span - 1) / span;
-  }
-  for (int rb = 0; rb < m; rb += Rm) {
-    const int i = rb + rl;
-    const bool live = i < m && gl < Gm;
-    const int ic = min(i, m - 1); /* idle lanes load row m - 1, unused */
-    V a0 = czero<V>();
-    double sx0 = 0, sy0 = 0, sx1 = 0, sy1 = 0;
-    for (int t = S.t0; t < S.t1; ++t) { /* identity terms */
-      const BfkTerm T = terms[t];
-      if (T.aOff >= 0 || !live || gl != 0) continue;
-      const V v = bufs.in[T.xbuf][T.xOff + i];
-      if constexpr (COMP) {
-        sx0 += (double)v.x;
-        sy0 += (double)v.y;
-      } else {
-        a0 = cadd(a0, v);
-      }
-    }
-    if (batches > 0) {
-      /* the load cursor: term ct, batch offset cj (uniform) */
-      int ct = S.t0; /* the first block term with columns (batches > 0: one exists) */
-      while (terms[ct].aOff < 0 || terms[ct].n <= 0) ++ct;
-      BfkTerm CT = terms[ct];
-      int cj = 0, issued = 0;
-      V xa[2][APPLY1_BATCH], aa[2][APPLY1_BATCH], la[2][APPLY1_BATCH];
-      int sn[2], sj[2];
-      auto issue = [&](int s) {
-        const V *x = bufs.in[CT.xbuf] + CT.xOff;
-        const int64_t ab = CT.aOff + CT.rowOff + ic, lda = CT.lda;
-        const int n = CT.n;
-#pragma unroll
-        for (int u = 0; u < APPLY1_BATCH; ++u) {
-          const int j = min(cj + gl + u * Gm, n - 1);
-          xa[s][u] = x[j];
-          aa[s][u] = hi[ab + (int64_t)j * lda];
-          if (LO) la[s][u] = lo[ab + (int64_t)j * lda];
-        }
-        sn[s] = n;
-        sj[s] = cj;
-        if (++issued < batches) { /* past the last batch the cursor stays put */
-          cj += span;
-          if (cj >= n) {
-            cj = 0;
-            do ++ct;
-            while (terms[ct].aOff < 0 || terms[ct].n <= 0);
-            CT = terms[ct];
-          }
-        }
-      };
-      auto compute = [&](int s) {
-#pragma unroll
-        for (int u = 0; u < APPLY1_BATCH; ++u) { /* selects, not branches: the loads stay above */
-          const bool ok = live && sj[s] + gl + u * Gm < sn[s];
-          if constexpr (COMP) {
-            double px, py;
-            if constexpr (LO) { /* hi + lo and the product in FP64: the pair's low part survives */
-              const double ar = (double)aa[s][u].x + (double)la[s][u].x;
-              const double ai = (double)aa[s][u].y + (double)la[s][u].y;
-              const double xr = (double)xa[s][u].x, xi = (double)xa[s][u].y;
-              px = fma(ar, xr, -ai * xi);
-              py = fma(ar, xi, ai * xr);
-            } else {
-              const V p = cmulf(aa[s][u], xa[s][u]);
-              px = (double)p.x;
-              py = (double)p.y;
-            }
-            px = ok ? px : 0.0;
-            py = ok ? py : 0.0;
-            if (u & 1) {
-              sx1 += px;
-              sy1 += py;
-            } else {
-              sx0 += px;
-              sy0 += py;
-            }
-          } else {
-            V t = cfmaT(aa[s][u], xa[s][u], a0);
-            if (LO) t = cfmaT(la[s][u], xa[s][u], t);
-            a0.x = ok ? t.x : a0.x;
-            a0.y = ok ? t.y : a0.y;
-          }
-        }
-      };
-      /* whole turns (two batches each), then the last batch if the count
-       * is odd: no exit inside a turn */
-      issue(0);
-      const int turns = batches >> 1;
-      for (int u = 0; u < turns; ++u) {
-        issue(1);
-        compute(0);
-        issue(0);
-        compute(1);
-      }
-      if (batches & 1) compute(0);
-    }
-    if constexpr (COMP) {
-      const double px = sx0 + sx1, py = sy0 + sy1;
-      double ax = px, ay = py;
-      for (int k = 1; k < Gm; ++k) { /* lanes rl + k Rm hold the other groups */
-        ax += __shfl(px, rl + k * Rm, 64);
-        ay += __shfl(py, rl + k * Rm, 64);
-      }
-      if (gl == 0 && i < m) {
-        V out;
-        out.x = (decltype(out.x))ax;
-        out.y = (decltype(out.y))ay;
-        y[i] = out;
-      }
-    } else {
-      V acc = a0;
-      for (int k = 1; k < Gm; ++k) {
-        acc.x += __shfl(a0.x, rl + k * Rm, 64);
-        acc.y += __shfl(a0.y, rl + k * Rm, 64);
-      }
-      if (gl == 0 && i < m) y[i] = acc;
-    }
-  }
-}
-
-#define APPLYN_ROWS 4
-
-__global__ __launch_bounds__(64) void k_applyN(const BfkSeg *__restrict__ segs, const BfkTerm *__restrict__ terms,
-                                               const double2 *__restrict__ arena, BfkBufs bufs, int nrhs) {
-  const BfkSeg S = segs[blockIdx.x];
-  const int c = blockIdx.y * 64 + threadIdx.x;
-  const bool live = c < nrhs;
-  const int m = S.m;
-  double2 *y = bufs.out[S.ybuf];
-  for (int rb = 0; rb < m; rb += APPLYN_ROWS) {
-    double2 acc[APPLYN_ROWS];
-    for (int q = 0; q < APPLYN_ROWS; ++q) acc[q] = make_double2(0, 0);
-    const int nr = min(APPLYN_ROWS, m - rb);
-    for (int t = S.t0; t < S.t1; ++t) {
-      const BfkTerm T = terms[t];
-      const double2 *x = bufs.in[T.xbuf];
-      if (T.aOff < 0) {
-        for (int q = 0; q < nr; ++q)
-          if (live) {
-            double2 v = x[(T.xOff + rb + q) * nrhs + c];
-            acc[q].x += v.x;
-            acc[q].y += v.y;
-          }
-      } else {
-        const double2 *A = arena + T.aOff + T.rowOff + rb;
-        const int64_t lda = T.lda;
-        for (int j = 0; j < T.n; ++j) {
-          double2 xv = live ? x[(T.xOff + j) * nrhs + c] : make_double2(0, 0);
-          for (int q = 0; q < nr; ++q) acc[q] = cfma(A[j * lda + q], xv, acc[q]);
-        }
-      }
-    }
-    if (live)
-      for (int q = 0; q < nr; ++q) y[(S.yOff + rb + q) * nrhs + c] = acc[q];
-  }
-}
 
 /* ------------------------------------------- many right-hand sides: MFMA */
 
@@ -2532,7 +2298,7 @@ int bfk_set_apply_config(int wavesPerBlock, int unroll, int mfmaTiles) {
                                             mfmaTiles == (8 | 16)))
     return -1;
   g_applyWaves = wavesPerBlock;
-  g_applyUnroll = unroll ? 1 : 0;
+  (void)unroll; /* the lane map follows the segment's height */
   g_mfmaCT = mfmaTiles;
   return 0;
 }
@@ -2930,36 +2696,26 @@ int bfk_ortho(const BfkOrthoJob *dJobs, const int32_t *dOrder, int numGroups, co
 }
 
 /* The launch shape of stage s: cfg < 0 takes the global settings; for one
- * right-hand side cfg = waves per block | unroll << 4, for 16 and more
+ * right-hand side cfg & 15 = segments per block, for 16 and more
  * cfg = right-hand-side tiles of 16 per MFMA wave | 16 for two row tiles
  * per wave (0 = the vector-unit kernel); between 2 and 15 right-hand sides
  * it is not used. */
 static int g_capturing = 0; /* launches go into a graph: no timing events */
 
-static int launch_stage_f64(const BfkSeg *segs, int64_t n, const BfkTerm *dTerms, const double *dArena,
-                            const BfkBufs &b, int nrhs, int cfg) {
+static int launch_stage_f64(const BfkSeg *segs, int64_t n, const BfkStageShape &shape, const BfkTerm *dTerms,
+                            const double *dArena, const BfkBufs &b, int nrhs, int cfg) {
   if (n == 0) return 0;
-  if (nrhs == 1) {
-    const int wv = cfg >= 0 ? (cfg & 15) : g_applyWaves;
-    const int unroll = cfg >= 0 ? (cfg >> 4) & 1 : g_applyUnroll;
-    dim3 grid((unsigned)((n + wv - 1) / wv)), block(64 * wv);
-    if (unroll)
-      hipLaunchKernelGGL((k_apply1<double2, false, true>), grid, block, 0, g_stream, segs, n, dTerms,
-                         (const double2 *)dArena, (const double2 *)nullptr, b);
-    else
-      hipLaunchKernelGGL((k_apply1<double2, false, false>), grid, block, 0, g_stream, segs, n, dTerms,
-                         (const double2 *)dArena, (const double2 *)nullptr, b);
-  } else if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
+  if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
     const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F64, nrhs);
     const int ct = mc & 15;
     const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
     dim3 grid(mfma_grid(n, chunks));
     launch_mfma<MfmaF64, false, false>(mc, grid, segs, dTerms, (const double2 *)dArena, nullptr, b, nrhs, chunks, n);
+    BFK_CHECK(hipGetLastError());
   } else {
-    hipLaunchKernelGGL(k_applyN, dim3((unsigned)n, (unsigned)((nrhs + 63) / 64)), dim3(64), 0, g_stream, segs,
-                       dTerms, (const double2 *)dArena, b, nrhs);
+    const int wv = nrhs == 1 && cfg >= 0 ? cfg & 15 : g_applyWaves;
+    BFK_CHECK(bfk_launch_few(g_stream, segs, n, shape, dTerms, (const double2 *)dArena, b, nrhs, wv));
   }
-  BFK_CHECK(hipGetLastError());
   return 0;
 }
 
@@ -2979,14 +2735,15 @@ static BfkBufs bufs_f64(const double *dX, double *dPing, double *dPong, double *
 /* one apply: `numStages` launches; stage s covers segments
  * [stageSeg[s], stageSeg[s+1]) with launch shape stageCfg[s] (NULL: the
  * global settings for every stage) */
-int bfk_apply(const BfkSeg *dSegs, const int64_t *stageSeg, int numStages, const BfkTerm *dTerms,
+int bfk_apply(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int numStages,
+              const BfkTerm *dTerms,
               const double *dArena, const double *dX, double *dPing, double *dPong, double *dY, int nrhs,
               const int32_t *stageCfg) {
   if (bfk_init()) return -1;
   const BfkBufs b = bufs_f64(dX, dPing, dPong, dY);
   if (!g_capturing && time_begin()) return -1;
   for (int s = 0; s < numStages; ++s)
-    if (launch_stage_f64(dSegs + stageSeg[s], stageSeg[s + 1] - stageSeg[s], dTerms, dArena, b, nrhs,
+    if (launch_stage_f64(dSegs + stageSeg[s], stageSeg[s + 1] - stageSeg[s], shapes[s], dTerms, dArena, b, nrhs,
                          stageCfg ? stageCfg[s] : -1))
       return -1;
   return g_capturing ? 0 : time_end(2);
@@ -2995,16 +2752,17 @@ int bfk_apply(const BfkSeg *dSegs, const int64_t *stageSeg, int numStages, const
 /* device ms per launch of stage s alone with launch shape cfg, averaged
  * over `reps` launches after one untimed launch (for the tuner; the
  * buffers hold whatever the last apply left) */
-int bfk_apply_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, int s, const BfkTerm *dTerms,
+int bfk_apply_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int s,
+                       const BfkTerm *dTerms,
                        const double *dArena, const double *dX, double *dPing, double *dPong, double *dY, int nrhs,
                        int cfg, int reps, double *ms) {
   if (bfk_init()) return -1;
   const BfkBufs b = bufs_f64(dX, dPing, dPong, dY);
   const int64_t n = stageSeg[s + 1] - stageSeg[s];
-  if (launch_stage_f64(dSegs + stageSeg[s], n, dTerms, dArena, b, nrhs, cfg)) return -1;
+  if (launch_stage_f64(dSegs + stageSeg[s], n, shapes[s], dTerms, dArena, b, nrhs, cfg)) return -1;
   BFK_CHECK(hipEventRecord(g_ev0, g_stream));
   for (int r = 0; r < reps; ++r)
-    if (launch_stage_f64(dSegs + stageSeg[s], n, dTerms, dArena, b, nrhs, cfg)) return -1;
+    if (launch_stage_f64(dSegs + stageSeg[s], n, shapes[s], dTerms, dArena, b, nrhs, cfg)) return -1;
   BFK_CHECK(hipEventRecord(g_ev1, g_stream));
   BFK_CHECK(hipEventSynchronize(g_ev1));
   float t = 0;
@@ -3048,7 +2806,7 @@ void bfk_graph_destroy(void *exec) {
 /* the global launch settings as one number: a captured apply is stale once
  * it changes */
 int bfk_apply_config_stamp(void) {
-  return g_applyWaves | g_applyUnroll << 4 | (g_mfmaCT & 31) << 5 | g_comp32 << 10 | g_foldMask << 14;
+  return g_applyWaves | (g_mfmaCT & 31) << 5 | g_comp32 << 10 | g_foldMask << 14;
 }
 
 int bfk_copy(const void *src, void *dst, size_t bytes) {
@@ -3104,45 +2862,6 @@ int bfk_lstsq_loaded(int64_t batch, int p, int n, const double *A, const double 
 
 /* ====================================================== FP32 apply path */
 
-__global__ __launch_bounds__(64) void k_applyN_f32(const BfkSeg *__restrict__ segs, const BfkTerm *__restrict__ terms,
-                                                   const float2 *__restrict__ hi, const float2 *__restrict__ lo,
-                                                   BfkBufsF bufs, int nrhs) {
-  const BfkSeg S = segs[blockIdx.x];
-  const int c = blockIdx.y * 64 + threadIdx.x;
-  const bool live = c < nrhs;
-  const int m = S.m;
-  float2 *y = bufs.out[S.ybuf];
-  for (int rb = 0; rb < m; rb += APPLYN_ROWS) {
-    float2 acc[APPLYN_ROWS];
-    for (int q = 0; q < APPLYN_ROWS; ++q) acc[q] = make_float2(0, 0);
-    const int nr = min(APPLYN_ROWS, m - rb);
-    for (int t = S.t0; t < S.t1; ++t) {
-      const BfkTerm T = terms[t];
-      const float2 *x = bufs.in[T.xbuf];
-      if (T.aOff < 0) {
-        for (int q = 0; q < nr; ++q)
-          if (live) {
-            float2 v = x[(T.xOff + rb + q) * nrhs + c];
-            acc[q].x += v.x;
-            acc[q].y += v.y;
-          }
-      } else {
-        const int64_t base = T.aOff + T.rowOff + rb;
-        const int64_t lda = T.lda;
-        for (int j = 0; j < T.n; ++j) {
-          float2 xv = live ? x[(T.xOff + j) * nrhs + c] : make_float2(0, 0);
-          for (int q = 0; q < nr; ++q) {
-            if (lo) acc[q] = cfmaf(lo[base + j * lda + q], xv, acc[q]);
-            acc[q] = cfmaf(hi[base + j * lda + q], xv, acc[q]);
-          }
-        }
-      }
-    }
-    if (live)
-      for (int q = 0; q < nr; ++q) y[(S.yOff + rb + q) * nrhs + c] = acc[q];
-  }
-}
-
 __global__ void k_to_f32(const double2 *__restrict__ a, int64_t n, float2 *__restrict__ hi, float2 *__restrict__ lo) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -3153,14 +2872,6 @@ __global__ void k_to_f32(const double2 *__restrict__ a, int64_t n, float2 *__res
     if (lo) lo[i] = make_float2((float)(v.x - (double)h.x), (float)(v.y - (double)h.y));
   }
 }
-
-template <bool LO, bool COMP>
-static void launch_apply1_f32(dim3 grid, dim3 block, const BfkSeg *segs, int64_t n, const BfkTerm *terms,
-                              const float2 *H, const float2 *Lo, BfkBufsF b) {
-  hipLaunchKernelGGL((k_apply1<float2, LO, false, COMP>), grid, block, 0, g_stream, segs, n, terms, H, Lo, b);
-}
-
-
 
 extern "C" {
 
@@ -3191,25 +2902,11 @@ int bfk_to_f32(const double *dArena, int64_t numEntries, float *dHi, float *dLo)
   return 0;
 }
 
-static int launch_stage_f32(const BfkSeg *segs, int64_t n, const BfkTerm *dTerms, const float *dArenaHi,
-                            const float *dArenaLo, const BfkBufsF &b, int nrhs, int cfg) {
+static int launch_stage_f32(const BfkSeg *segs, int64_t n, const BfkStageShape &shape, const BfkTerm *dTerms,
+                            const float *dArenaHi, const float *dArenaLo, const BfkBufsF &b, int nrhs, int cfg) {
   if (n == 0) return 0;
   const float2 *H = (const float2 *)dArenaHi, *Lo = (const float2 *)dArenaLo;
-  if (nrhs == 1) {
-    const int wv = cfg >= 0 ? (cfg & 15) : g_applyWaves;
-    const int unroll = cfg >= 0 ? (cfg >> 4) & 1 : g_applyUnroll;
-    dim3 grid((unsigned)((n + wv - 1) / wv)), block(64 * wv);
-    if (g_comp32) {
-      if (Lo) launch_apply1_f32<true, true>(grid, block, segs, n, dTerms, H, Lo, b);
-      else launch_apply1_f32<false, true>(grid, block, segs, n, dTerms, H, Lo, b);
-    } else if (Lo) {
-      launch_apply1_f32<true, false>(grid, block, segs, n, dTerms, H, Lo, b);
-    } else if (unroll) {
-      hipLaunchKernelGGL((k_apply1<float2, false, true>), grid, block, 0, g_stream, segs, n, dTerms, H, Lo, b);
-    } else {
-      launch_apply1_f32<false, false>(grid, block, segs, n, dTerms, H, Lo, b);
-    }
-  } else if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
+  if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
     const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F32, nrhs);
     const int ct = mc & 15;
     const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
@@ -3222,11 +2919,11 @@ static int launch_stage_f32(const BfkSeg *segs, int64_t n, const BfkTerm *dTerms
       if (g_comp32) launch_mfma<MfmaF32, false, true>(mc, grid, segs, dTerms, H, Lo, b, nrhs, chunks, n);
       else launch_mfma<MfmaF32, false, false>(mc, grid, segs, dTerms, H, Lo, b, nrhs, chunks, n);
     }
+    BFK_CHECK(hipGetLastError());
   } else {
-    hipLaunchKernelGGL(k_applyN_f32, dim3((unsigned)n, (unsigned)((nrhs + 63) / 64)), dim3(64), 0, g_stream, segs,
-                       dTerms, H, Lo, b, nrhs);
+    const int wv = nrhs == 1 && cfg >= 0 ? cfg & 15 : g_applyWaves;
+    BFK_CHECK(bfk_launch_few_f32(g_stream, segs, n, shape, dTerms, H, Lo, b, nrhs, wv, g_comp32 != 0));
   }
-  BFK_CHECK(hipGetLastError());
   return 0;
 }
 
@@ -3243,29 +2940,31 @@ static BfkBufsF bufs_f32(const float *dX, float *dPing, float *dPong, float *dY)
   return b;
 }
 
-int bfk_apply_f32(const BfkSeg *dSegs, const int64_t *stageSeg, int numStages, const BfkTerm *dTerms,
+int bfk_apply_f32(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int numStages,
+                  const BfkTerm *dTerms,
                   const float *dArenaHi, const float *dArenaLo, const float *dX, float *dPing, float *dPong, float *dY,
                   int nrhs, const int32_t *stageCfg) {
   if (bfk_init()) return -1;
   const BfkBufsF b = bufs_f32(dX, dPing, dPong, dY);
   if (!g_capturing && time_begin()) return -1;
   for (int s = 0; s < numStages; ++s)
-    if (launch_stage_f32(dSegs + stageSeg[s], stageSeg[s + 1] - stageSeg[s], dTerms, dArenaHi, dArenaLo, b, nrhs,
+    if (launch_stage_f32(dSegs + stageSeg[s], stageSeg[s + 1] - stageSeg[s], shapes[s], dTerms, dArenaHi, dArenaLo, b, nrhs,
                          stageCfg ? stageCfg[s] : -1))
       return -1;
   return g_capturing ? 0 : time_end(3);
 }
 
-int bfk_apply_f32_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, int s, const BfkTerm *dTerms,
+int bfk_apply_f32_stage_ms(const BfkSeg *dSegs, const int64_t *stageSeg, const BfkStageShape *shapes, int s,
+                           const BfkTerm *dTerms,
                            const float *dArenaHi, const float *dArenaLo, const float *dX, float *dPing, float *dPong,
                            float *dY, int nrhs, int cfg, int reps, double *ms) {
   if (bfk_init()) return -1;
   const BfkBufsF b = bufs_f32(dX, dPing, dPong, dY);
   const int64_t n = stageSeg[s + 1] - stageSeg[s];
-  if (launch_stage_f32(dSegs + stageSeg[s], n, dTerms, dArenaHi, dArenaLo, b, nrhs, cfg)) return -1;
+  if (launch_stage_f32(dSegs + stageSeg[s], n, shapes[s], dTerms, dArenaHi, dArenaLo, b, nrhs, cfg)) return -1;
   BFK_CHECK(hipEventRecord(g_ev0, g_stream));
   for (int r = 0; r < reps; ++r)
-    if (launch_stage_f32(dSegs + stageSeg[s], n, dTerms, dArenaHi, dArenaLo, b, nrhs, cfg)) return -1;
+    if (launch_stage_f32(dSegs + stageSeg[s], n, shapes[s], dTerms, dArenaHi, dArenaLo, b, nrhs, cfg)) return -1;
   BFK_CHECK(hipEventRecord(g_ev1, g_stream));
   BFK_CHECK(hipEventSynchronize(g_ev1));
   float t = 0;

@@ -81,6 +81,13 @@ typedef struct BfkTerm {
   int32_t xbuf;
 } BfkTerm;
 
+/* What the launch of a stage goes by: the columns of its terms summed over
+ * its segments, and the height of its tallest segment. */
+typedef struct BfkStageShape {
+  int64_t cols;
+  int32_t maxRows, pad;
+} BfkStageShape;
+
 /* Orthogonalization of a butterfly (a change of basis of every
  * intermediate vector; the operator is unchanged).  One job is one column
  * block of one factor: its blocks (items [i0, i1)) are first multiplied on

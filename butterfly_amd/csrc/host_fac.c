@@ -44,6 +44,8 @@ static void free_plan(BfMatHipButterfly *F) {
   BF_VEC_FREE(F->segs);
   BF_VEC_FREE(F->terms);
   BF_VEC_FREE(F->stageSeg);
+  free(F->stageShape);
+  F->stageShape = NULL;
 }
 
 static void free_device(BfMatHipButterfly *F) {
@@ -102,6 +104,34 @@ static int cmp_i64(const void *a, const void *b) {
 }
 
 static int32_t stage_buf(int s) { return (s % 2 == 0) ? BFK_BUF_PING : BFK_BUF_PONG; }
+
+/* The next term of the segment whose terms start at t0.  The blocks of a
+ * factor's row lie one after another in the arena and, unless an identity
+ * stands between them, so do the inputs they read: such a term only makes
+ * the one before it wider. */
+static inline void push_term(BfMatHipButterfly *F, int32_t t0, BfkTerm t) {
+  if (F->terms.n > (size_t)t0) {
+    BfkTerm *p = &F->terms.a[F->terms.n - 1];
+    if (p->aOff >= 0 && t.aOff == p->aOff + (int64_t)p->lda * p->n && t.lda == p->lda && t.rowOff == p->rowOff &&
+        t.xbuf == p->xbuf && t.xOff == p->xOff + p->n && (int64_t)p->n + t.n <= INT32_MAX) {
+      p->n += t.n;
+      return;
+    }
+  }
+  BF_VEC_PUSH(F->terms, t);
+}
+
+BfkStageShape *bfStageShapes(const BfkSeg *segs, const int64_t *stageSeg, int numStages, const BfkTerm *terms) {
+  BfkStageShape *sh = calloc((size_t)(numStages > 0 ? numStages : 1), sizeof(BfkStageShape));
+  if (!sh) return NULL;
+  for (int s = 0; s < numStages; ++s)
+    for (int64_t i = stageSeg[s]; i < stageSeg[s + 1]; ++i) {
+      if (segs[i].m > sh[s].maxRows) sh[s].maxRows = segs[i].m;
+      for (int32_t t = segs[i].t0; t < segs[i].t1; ++t)
+        if (terms[t].aOff >= 0) sh[s].cols += terms[t].n;
+    }
+  return sh;
+}
 
 /* Stage layout: butterfly b with nf factors runs factor f at stage
  * Fmax - nf + f, so every last factor and every dense leaf lands in the
@@ -185,7 +215,7 @@ int bfApplyPlanBuild(BfMatHipButterfly *F) {
             t.xbuf = stage_buf(s - 1);
           }
           if (bl->dataOff >= 0) facBytes += 16.0 * bl->m * bl->n;
-          BF_VEC_PUSH(F->terms, t);
+          push_term(F, sg.t0, t);
         }
         sg.t1 = (int32_t)F->terms.n;
         BF_VEC_PUSH(F->segs, sg);
@@ -288,6 +318,8 @@ int bfApplyPlanBuild(BfMatHipButterfly *F) {
     BF_VEC_PUSH(F->segs, sg);
   }
   BF_VEC_PUSH(F->stageSeg, (int64_t)F->segs.n);
+  free(F->stageShape);
+  F->stageShape = bfStageShapes(F->segs.a, F->stageSeg.a, F->numStages, F->terms.a);
   F->applyFactorBytes = facBytes;
   F->stats[11] = facBytes;
   F->stats[12] = vecBytes;
@@ -297,7 +329,7 @@ int bfApplyPlanBuild(BfMatHipButterfly *F) {
   BF_VEC_FREE(cons);
   free(fill);
   free(region);
-  if (F->terms.n > (size_t)INT32_MAX) return -1;
+  if (F->terms.n > (size_t)INT32_MAX || !F->stageShape) return -1;
   return 0;
 }
 
@@ -1114,9 +1146,9 @@ int bfhipSetApplyGraphs(int on) {
 static int enqueue_apply(BfMatHipButterfly *F, void const *dX, void *dY, BfSize nrhs, BfhipPrecision prec,
                          const int32_t *cfg) {
   if (prec == BFHIP_PRECISION_FP64)
-    return bfk_apply(F->dSegs, F->stageSeg.a, F->numStages, F->dTerms, F->dArena, dX, F->dPing, F->dPong, dY,
+    return bfk_apply(F->dSegs, F->stageSeg.a, F->stageShape, F->numStages, F->dTerms, F->dArena, dX, F->dPing, F->dPong, dY,
                      (int)nrhs, cfg);
-  return bfk_apply_f32(F->dSegs, F->stageSeg.a, F->numStages, F->dTerms, F->dArena32,
+  return bfk_apply_f32(F->dSegs, F->stageSeg.a, F->stageShape, F->numStages, F->dTerms, F->dArena32,
                        prec == BFHIP_PRECISION_FP32X2 ? F->dArena32lo : NULL, dX, F->dPing, F->dPong, dY, (int)nrhs,
                        cfg);
 }
@@ -1224,11 +1256,11 @@ int bfhipFacTuneApply(BfMat *fac, BfSize nrhs, BfhipPrecision prec, char const *
   const int cls = bf_nrhs_class(nrhs);
   if (cls == 1) return 0; /* 2-15 right-hand sides: the vector-unit kernel only */
   if (!cachePath) cachePath = getenv("BF_AMD_TUNE_CACHE");
-  /* candidates: waves per block x lane map (1 RHS); tiles per MFMA wave
-   * x one or two row tiles, 0 = the vector-unit kernel (16 and more) */
-  static const int one[] = {1, 2, 4, 1 | 16, 2 | 16, 4 | 16}, many[] = {1, 2, 4, 8, 1 | 16, 2 | 16, 4 | 16, 0};
+  /* candidates: segments per block (1 RHS); tiles per MFMA wave x one or
+   * two row tiles, 0 = the vector-unit kernel (16 and more) */
+  static const int one[] = {1, 2, 4}, many[] = {1, 2, 4, 8, 1 | 16, 2 | 16, 4 | 16, 0};
   const int *cand = cls == 0 ? one : many;
-  const int nc = cls == 0 ? 6 : 8;
+  const int nc = cls == 0 ? 3 : 8;
   const size_t elem = prec == BFHIP_PRECISION_FP64 ? 16 : 8;
   int rc = ensure_buffers(F, nrhs, elem);
   void *dX = rc ? NULL : bfk_malloc(F->numSrc * nrhs * elem + 16);
@@ -1254,9 +1286,9 @@ int bfhipFacTuneApply(BfMat *fac, BfSize nrhs, BfhipPrecision prec, char const *
     for (int c = 0; c < nc && !rc; ++c) {
       double ms = 0;
       rc = prec == BFHIP_PRECISION_FP64
-               ? bfk_apply_stage_ms(F->dSegs, F->stageSeg.a, s, F->dTerms, F->dArena, dX, F->dPing, F->dPong, dY,
+               ? bfk_apply_stage_ms(F->dSegs, F->stageSeg.a, F->stageShape, s, F->dTerms, F->dArena, dX, F->dPing, F->dPong, dY,
                                     (int)nrhs, cand[c], 3, &ms)
-               : bfk_apply_f32_stage_ms(F->dSegs, F->stageSeg.a, s, F->dTerms, F->dArena32,
+               : bfk_apply_f32_stage_ms(F->dSegs, F->stageSeg.a, F->stageShape, s, F->dTerms, F->dArena32,
                                         prec == BFHIP_PRECISION_FP32X2 ? F->dArena32lo : NULL, dX, F->dPing,
                                         F->dPong, dY, (int)nrhs, cand[c], 3, &ms);
       if (!rc && ms < best) {
@@ -1325,9 +1357,9 @@ int bfhipMatMulDeviceNoAlloc(BfMat const *fac, void const *dX, void *dY, BfSize 
   int rc;
   const int32_t *cfg = F->tuneCfg[prec][bf_nrhs_class(nrhs)];
   if (prec == BFHIP_PRECISION_FP64)
-    rc = bfk_apply(F->dSegs, F->stageSeg.a, F->numStages, F->dTerms, F->dArena, dX, ping, pong, dY, (int)nrhs, cfg);
+    rc = bfk_apply(F->dSegs, F->stageSeg.a, F->stageShape, F->numStages, F->dTerms, F->dArena, dX, ping, pong, dY, (int)nrhs, cfg);
   else
-    rc = bfk_apply_f32(F->dSegs, F->stageSeg.a, F->numStages, F->dTerms, F->dArena32,
+    rc = bfk_apply_f32(F->dSegs, F->stageSeg.a, F->stageShape, F->numStages, F->dTerms, F->dArena32,
                        prec == BFHIP_PRECISION_FP32X2 ? F->dArena32lo : NULL, dX, ping, pong, dY, (int)nrhs, cfg);
   if (rc) bfSetError(BF_ERROR_RUNTIME_ERROR);
   return rc;

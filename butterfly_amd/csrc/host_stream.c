@@ -1300,6 +1300,7 @@ typedef struct BfMatHipProduct {
   BfSegVec segs;
   BfTermVec terms;
   BfI64Vec stageSeg;
+  BfkStageShape *stageShape;
   int numStages;
   int64_t bufRows;
   int64_t entries;
@@ -1322,6 +1323,7 @@ static void prod_delete(BfMat **mp) {
   BF_VEC_FREE(P->segs);
   BF_VEC_FREE(P->terms);
   BF_VEC_FREE(P->stageSeg);
+  free(P->stageShape);
   free(P);
   *mp = NULL;
 }
@@ -1407,6 +1409,8 @@ static BfMat *product_new(const SMat *const *F, size_t nf) {
   }
   BF_VEC_PUSH(P->stageSeg, (int64_t)P->segs.n);
   int rc = 0;
+  P->stageShape = bfStageShapes(P->segs.a, P->stageSeg.a, P->numStages, P->terms.a);
+  if (!P->stageShape) rc = -2;
   P->dArena = bfk_malloc((size_t)(entries ? entries : 1) * 16);
   P->dSegs = bfk_malloc((P->segs.n ? P->segs.n : 1) * sizeof(BfkSeg));
   P->dTerms = bfk_malloc((P->terms.n ? P->terms.n : 1) * sizeof(BfkTerm));
@@ -1452,7 +1456,7 @@ static BfMat *prod_mul(BfMat const *A, BfMat const *Xm) {
   if (!dx || !dy) rc = -2;
   if (!rc) rc = bfk_h2d(dx, hx, (size_t)(n * nrhs) * 16);
   if (!rc)
-    rc = bfk_apply(P->dSegs, P->stageSeg.a, P->numStages, P->dTerms, P->dArena, dx, P->dPing, P->dPong, dy,
+    rc = bfk_apply(P->dSegs, P->stageSeg.a, P->stageShape, P->numStages, P->dTerms, P->dArena, dx, P->dPing, P->dPong, dy,
                    (int)nrhs, NULL);
   BfMatDenseComplex *Y = NULL;
   if (!rc) {

@@ -492,9 +492,9 @@ void bfhipGetKernelTimes(double out[8]);
 void bfhipGetKernelTimeSums(double sums[8], double counts[8]);
 void bfhipResetKernelTimes(void);
 /* new: launch shapes of the apply, for tuning: the 1-RHS apply's waves per
- * block in {1, 2, 4} (one row segment per wave) and, when `unroll` is 1,
- * the power-of-two lane map instead of the default map whose rows match
- * the segment height; the many-RHS apply's right-hand-side
+ * block in {1, 2, 4} (one row segment per wave where segments are not split
+ * over waves; `unroll` is accepted and has no effect: the lane map follows
+ * the segment's height); the many-RHS apply's right-hand-side
  * tiles of 16 per wave on the matrix cores in {1, 2, 4, 8}, plus 16 for
  * two 16-row tiles per wave (tiles 1, 2 or 4), 0 for the vector-unit
  * kernel, or -1 (the default: the shapes the tuner picks at N = 2^20, 2
@@ -520,7 +520,7 @@ int bfhipSetApplyGraphs(int on);
 void bfhipSetLstsqWaves(int64_t twoAbove, int64_t fourAbove, int64_t *oldTwo, int64_t *oldFour);
 /* new (no counterpart): the apply's autotuner.  For each apply stage of
  * `fac` it times the launch shapes that fit `nrhs` (one right-hand side:
- * 1, 2 or 4 waves per block with either lane map; 16 and more: 1, 2, 4 or
+ * 1, 2 or 4 segments per block; 16 and more: 1, 2, 4 or
  * 8 tiles of 16 right-hand sides per matrix-core wave, 1, 2 or 4 with two
  * row tiles per wave, or the vector-unit kernel) on that stage alone and keeps the fastest, per bucket of stages
  * (rounded log2 of the mean segment height and of the mean columns per
