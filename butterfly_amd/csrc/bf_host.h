@@ -36,6 +36,8 @@ int bfk_sketch_project(int64_t batch, const void *dJobs, const int64_t *dSOff, c
 size_t bfk_lstsq_lds_bytes(int p, int n);
 void *bfk_malloc(size_t bytes);
 void bfk_free(void *p);
+void *bfk_host_malloc(size_t bytes); /* page-locked */
+void bfk_host_free(void *p);
 void bfk_free_async(void *p);
 int bfk_h2d(void *dst, const void *src, size_t bytes);
 int bfk_h2d_side(void *dst, const void *src, size_t bytes);
@@ -61,15 +63,17 @@ int bfk_bie_post(int64_t n, int nrhs, int ncorr, double alpha, const int32_t *dC
 int bfk_dotc_multi(int64_t n, int nv, const double *dV, int64_t ldv, const double *dW, double *hOut);
 int bfk_axpy_multi(int64_t n, int nv, const double *dV, int64_t ldv, const double *hH, double s, double *dW);
 int bfk_convert(int64_t n, const void *src, void *dst, int to32);
-int bfk_svd_jacobi(int64_t batch, const int64_t *dAOff, const int32_t *dM, const int32_t *dN, double *dA,
-                   const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, int maxSweeps);
+int bfk_svd_jacobi(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,
+                   double *dA, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, int maxSweeps);
 int bfk_svd_jacobi_big(int64_t nb, const int32_t *dBig, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,
                        double *dA, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig,
                        int maxSweeps, int maxN);
 int bfk_svd_tall_max_n(void);
-int bfk_svd_jacobi_tall(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,
-                        double *dA, double *dS, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig,
-                        int maxSweeps, int maxN);
+int bfk_svd_qr_max_n(void);
+size_t bfk_svd_qr_scratch(int64_t nb, int maxN);
+int bfk_svd_qr(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN, double *dA,
+               double *dS, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, void *dWork,
+               int maxSweeps, int maxN);
 size_t bfk_ortho_units(int rows, int n);
 int bfk_ortho(const BfkOrthoJob *dJobs, const int32_t *dOrder, int numGroups, const int64_t *groupStart,
               const size_t *groupBytes, const BfkOrthoItem *dItems, double *dArena, const double *dRin,

@@ -364,8 +364,9 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
  * for blk_sum).  A rotation of
  * rows i < j with g = r_i . conj(r_j), a = |r_i|^2, b = |r_j|^2:
  *   e = g/|g|, zeta = (b - a)/(2|g|), t = sign(zeta)/(|zeta| + sqrt(1 + zeta^2)),
- *   c = 1/sqrt(1 + t^2), s = c t;  r_i <- c r_i - s e r_j,  r_j <- s r_i + c e r_j. */
-template <int LP, int G>
+ *   c = 1/sqrt(1 + t^2), s = c t;  r_i <- c r_i - s e r_j,  r_j <- s r_i + c e r_j.
+ * With EXACT (the SVDs) sweeps go on until one rotates nothing. */
+template <int LP, int G, bool EXACT = false>
 __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int W, int ld, double *red) {
   const int lane = threadIdx.x;
   const double eps = 2.220446049250313e-16;
@@ -479,7 +480,7 @@ __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int 
      * to about 1e-12 relative, an order under the 1e-11 singular-value cut,
      * so the next sweep, which would move singular values and vectors by
      * that much, is skipped */
-    if (!blk_any<G>(big, red)) break;
+    if (!EXACT && !blk_any<G>(big, red)) break;
   }
 }
 
@@ -979,21 +980,26 @@ __global__ void k_f32_to_f64(int64_t n, const float2 *__restrict__ a, double2 *_
 
 /* ------------------------------------------------ batched one-sided SVD */
 
-/* Singular value decomposition of a batch of m x n complex matrices
- * (column-major, m >= 1, n >= 1; the host keeps n <= 1024, as the work grows
- * with n^2), one 256-thread block each, in
- * place: one-sided (Hestenes) Jacobi rotates pairs of columns until they
- * are orthogonal, A V = W with orthogonal columns w_j = sigma_j u_j.  On
- * return A holds W, V (n x n, column-major) the accumulated rotations and
- * sig[j] = |w_j|.  Pairs follow the round-robin order, one group of g
- * threads per pair (g a power of two <= 64, so a pair's reduction stays
- * in one wave). */
-__global__ __launch_bounds__(256) void k_svd_jacobi(const int64_t *__restrict__ aOff, const int32_t *__restrict__ mm,
-                                                    const int32_t *__restrict__ nn, double2 *__restrict__ A,
+/* Singular value decompositions of m x n complex matrices (column-major,
+ * m >= n) by one-sided (Hestenes) Jacobi: pairs of columns, or of rows of
+ * the triangle a QR leaves, are rotated until all are orthogonal, A V = W
+ * with orthogonal columns w_j = sigma_j u_j.  On return A holds W, V (n x n,
+ * column-major) the rotations and sig[j] = |w_j|.
+ *
+ * k_svd_jacobi rotates the columns in global memory, one 256-thread
+ * workgroup per matrix, one group of g threads per pair (g a power of two
+ * <= 64, so a pair's reduction stays in one wave).  It is left for the
+ * matrices of more than 256 rows and less than 2^15 entries: through their
+ * QR they would take a quarter of the time, but their ranks in a stream are
+ * decided by singular values that rounding moves by 1% (bases known to
+ * 1e-8 merge at a cut of 1e-8), and the factor shapes that streams of such
+ * blocks have given stay what they are. */
+__global__ __launch_bounds__(256) void k_svd_jacobi(const int32_t *__restrict__ idx, const int64_t *__restrict__ aOff,
+                                                    const int32_t *__restrict__ mm, const int32_t *__restrict__ nn, double2 *__restrict__ A,
                                                     const int64_t *__restrict__ vOff, double2 *__restrict__ V,
                                                     const int64_t *__restrict__ sOff, double *__restrict__ sig,
                                                     int maxSweeps) {
-  const int b = blockIdx.x;
+  const int b = idx[blockIdx.x];
   const int m = mm[b], n = nn[b];
   double2 *a = A + aOff[b];
   double2 *v = V + vOff[b];
@@ -1077,13 +1083,12 @@ __global__ __launch_bounds__(256) void k_svd_jacobi(const int64_t *__restrict__ 
   }
 }
 
-/* The same Jacobi for large matrices, spread over the chip: one launch per
- * round-robin step, workgroup (p, b) rotates pair p of big matrix b with
- * 256 threads over the rows (block reductions), so a step of a matrix with
- * 300 pairs uses 300 workgroups instead of one.  Pairs, order, rotation
- * and stopping rule are those of k_svd_jacobi; a matrix whose `active`
- * flag is 0 (no rotation in its previous sweep) is skipped, and every
- * rotation sets rot[b]. */
+/* Matrices of more than SVD_QR_MAX_N columns: the same rotations spread over
+ * the chip, one launch per round-robin step, workgroup (p, b) rotates pair p
+ * of matrix b with 256 threads over the rows (block reductions), so a step
+ * of a matrix with 300 pairs uses 300 workgroups instead of one.  A matrix
+ * whose `active` flag is 0 (no rotation in its previous sweep) is skipped,
+ * and every rotation sets rot[b]. */
 __global__ __launch_bounds__(256) void k_svd_step(const int32_t *__restrict__ big, const int64_t *__restrict__ aOff,
                                                   const int32_t *__restrict__ mm, const int32_t *__restrict__ nn,
                                                   double2 *__restrict__ A, const int64_t *__restrict__ vOff,
@@ -1228,38 +1233,174 @@ __device__ __forceinline__ double house_apply_wave(const double2 *__restrict__ x
   return NORM ? group_sum(nq, 64) : 0.0;
 }
 
-/* SVD of a tall matrix (m >= 2n, n <= SVD_TALL_MAX_N), in three launches:
+/* SVD of a matrix of at most SVD_QR_MAX_N columns, through its triangle:
  *   k_tall_qr      Householder QR with column pivoting of a copy S of A
  *                  (global memory; each wave takes every 16th column of a
  *                  step), A P = Q R; R, the pivots and the reflectors' scales
  *                  go to a per-matrix scratch slot
- *   k_tall_jacobi  one wave: one-sided Jacobi on the rows of [R | I] in LDS
- *                  (jacobi_rows, as for the re-expansion blocks): G R = R'
- *                  with orthogonal rows sigma_i v_i^H, G accumulated
+ *   k_tall_jacobi  (n <= SVD_TALL_MAX_N) one workgroup: one-sided Jacobi on
+ *                  the rows of [R | I] in LDS (jacobi_rows, as for the
+ *                  re-expansion blocks): G R = R' with orthogonal rows
+ *                  sigma_i v_i^H, G accumulated
+ *   k_svd_block    (wider) the same on blocks of rows, a workgroup per pair
+ *                  of blocks, a launch per round
  *   k_tall_w       sigma_i = |row i of R'|, V = P [conj(R') / sigma]^T, and
- *                  W = Q [sigma_i conj(G[i, :]); 0] with Q in compact WY
- *                  form (one pass over the reflectors), so A V = W and W's
+ *                  W = Q [sigma_i conj(G[i, :]); 0], so A V = W and W's
  *                  columns keep their mutual orthogonality relative to
- *                  their own norms
+ *                  their own norms: Q in compact WY form (one pass over the
+ *                  reflectors), or for the wider ones (k_wide_w) one
+ *                  reflector after the other, a wave per column
  * The pivoted QR grades R's rows, so the row Jacobi needs few sweeps; the
- * rotations touch n-row operands instead of m. */
+ * rotations touch n-row operands instead of m.  Bound: the LDS traffic of a
+ * Jacobi step (a step of 30 pairs of 120 entries moves 290 KB: 2300 of a
+ * CU's clocks), in a chain of n - 1 steps a sweep; rotating the columns of
+ * A itself, in global memory by one workgroup, took 12 ms for 256 x 60 where
+ * this takes 0.9, and 85 ms for 256 x 180 where this takes 3. */
 #define SVD_TALL_MAX_N 70
-#define SVD_TALL_T 1024 /* threads of the QR and W launches */
+#define SVD_QR_MAX_N 256
+#define SVD_TALL_T 1024 /* threads of the QR, Jacobi and W launches */
 __host__ __device__ __forceinline__ int tall_ld(int n) { return 2 * n + 1; }
-__host__ __device__ __forceinline__ size_t svd_tall_lds(int n) { return (size_t)n * tall_ld(n) * 16; }
+/* [R | I] and the reductions of 16 waves */
+__host__ __device__ __forceinline__ size_t svd_tall_lds(int n) { return (size_t)n * tall_ld(n) * 16 + 256; }
 __host__ __device__ __forceinline__ size_t svd_tall_w_lds(int n) { return (size_t)2 * n * n * 16; }
-/* scratch slot of one matrix: [R | I] then [R' | G], n x (2n + 1) */
-#define TALL_SLOT ((int64_t)SVD_TALL_MAX_N * (2 * SVD_TALL_MAX_N + 1))
+/* scratch slot of one matrix of a batch whose widest has maxN columns:
+ * [R | I] then [R' | G], n x (2n + 1) */
+static inline int64_t tall_slot(int maxN) { return (int64_t)maxN * (2 * maxN + 1); }
+
+/* The QR with the matrix in registers: wave w holds columns w, w + 16, ...
+ * (CPW of them, RPL rows a lane), so a step costs one broadcast of the
+ * reflector through LDS and the arithmetic on what is left, where the same
+ * step in global memory waits for two passes through L2 (256 x 60: 240 us
+ * -> 60 us).  Columns stay where they are: pos[c] is the step that took
+ * column c, and row i of a column not yet taken is final after step i. */
+template <int RPL, int CPW>
+__device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *__restrict__ s, int m, int n,
+                                        double2 *__restrict__ rg, int32_t *__restrict__ piv, double *__restrict__ hinv,
+                                        double *__restrict__ cn, int *__restrict__ pos, double2 *__restrict__ v) {
+  constexpr int NW = SVD_TALL_T / 64;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  double2 x[CPW][RPL];
+#pragma unroll
+  for (int q = 0; q < CPW; ++q) {
+    const int c = w + NW * q;
+    double nq = 0;
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) {
+      const int r = lane + 64 * u;
+      x[q][u] = c < n && r < m ? a[(int64_t)c * m + r] : make_double2(0, 0);
+      nq = fma(x[q][u].x, x[q][u].x, fma(x[q][u].y, x[q][u].y, nq));
+    }
+    nq = group_sum(nq, 64);
+    if (lane == 0 && c < n) {
+      cn[c] = nq;
+      pos[c] = -1; /* not taken */
+    }
+  }
+  __syncthreads();
+  double2 diag[CPW]; /* the diagonal of R in the columns taken */
+#pragma unroll
+  for (int q = 0; q < CPW; ++q) diag[q] = make_double2(0, 0);
+  for (int j = 0; j < n; ++j) {
+    /* the largest remaining column, the first among equals; where no
+     * comparison holds (NaN) the first remaining one */
+    double best = -1.0;
+    int bi = n, free1 = n;
+    for (int c = lane; c < n; c += 64)
+      if (pos[c] < 0) {
+        free1 = min(free1, c);
+        if (cn[c] > best) { best = cn[c]; bi = c; }
+      }
+    wave_argmax(best, bi);
+    for (int o = 32; o > 0; o >>= 1) free1 = min(free1, __shfl_xor(free1, o, 64));
+    const int p = __builtin_amdgcn_readfirstlane(bi < n ? bi : free1);
+    const double sg = sqrt(cn[p]);
+    if (w == (p & (NW - 1))) { /* the wave that holds it: the reflector */
+#pragma unroll
+      for (int q = 0; q < CPW; ++q)
+        if (q == p / NW) {
+          double2 x0 = make_double2(0, 0);
+#pragma unroll
+          for (int u = 0; u < RPL; ++u)
+            if (u == (j >> 6)) x0 = make_double2(__shfl(x[q][u].x, j & 63, 64), __shfl(x[q][u].y, j & 63, 64));
+          const double ax0 = hypot(x0.x, x0.y);
+          const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;
+          diag[q] = sg > 0 ? make_double2(-phx * sg, -phy * sg) : x0;
+#pragma unroll
+          for (int u = 0; u < RPL; ++u) {
+            const int r = lane + 64 * u;
+            double2 y = r < j ? make_double2(0, 0) : x[q][u];
+            if (r == j && sg > 0) y = make_double2(x0.x + phx * sg, x0.y + phy * sg);
+            v[r] = y;
+            if (r < m) s[(int64_t)j * m + r] = y;
+          }
+          if (lane == 0) {
+            const double inv = sg > 0 ? 1.0 / (sg * (sg + ax0)) : 0.0;
+            hinv[j] = inv;
+            v[64 * RPL].x = inv;
+            piv[j] = p;
+          }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) pos[p] = j;
+    const double inv = v[64 * RPL].x;
+    double2 vv[RPL];
+#pragma unroll
+    for (int u = 0; u < RPL; ++u) vv[u] = v[lane + 64 * u];
+#pragma unroll
+    for (int q = 0; q < CPW; ++q) {
+      const int c = w + NW * q;
+      if (c < n && c != p && pos[c] < 0) { /* uniform; pos[p] may or may not be set yet */
+        double dx = 0, dy = 0, nq = 0;
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) {
+          dx = fma(vv[u].x, x[q][u].x, fma(vv[u].y, x[q][u].y, dx));
+          dy = fma(vv[u].x, x[q][u].y, fma(-vv[u].y, x[q][u].x, dy));
+        }
+        dx = group_sum(dx, 64) * inv;
+        dy = group_sum(dy, 64) * inv;
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) { /* without a reflector inv = 0: only the norm moves on */
+          x[q][u].x -= vv[u].x * dx - vv[u].y * dy;
+          x[q][u].y -= vv[u].x * dy + vv[u].y * dx;
+          if (lane + 64 * u > j) nq = fma(x[q][u].x, x[q][u].x, fma(x[q][u].y, x[q][u].y, nq));
+        }
+        nq = group_sum(nq, 64);
+        if (lane == 0) cn[c] = nq;
+      }
+    }
+    __syncthreads();
+  }
+  /* [R | I], row-major with leading dimension 2n + 1 */
+  const int ld = tall_ld(n);
+#pragma unroll
+  for (int q = 0; q < CPW; ++q) {
+    const int c = w + NW * q;
+    if (c < n) {
+      const int p = pos[c];
+#pragma unroll
+      for (int u = 0; u < RPL; ++u) {
+        const int r = lane + 64 * u;
+        if (r < n) rg[r * ld + p] = r < p ? x[q][u] : r == p ? diag[q] : make_double2(0, 0);
+      }
+    }
+  }
+  for (int e = tid; e < n * n; e += SVD_TALL_T) {
+    const int i = e / n, c = e - i * n;
+    rg[i * ld + n + c] = make_double2(c == i ? 1.0 : 0.0, 0.0);
+  }
+}
 
 __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restrict__ idx,
                                                         const int64_t *__restrict__ aOff,
                                                         const int32_t *__restrict__ mm,
                                                         const int32_t *__restrict__ nn, const double2 *__restrict__ A,
                                                         double2 *__restrict__ S, double2 *__restrict__ RG,
-                                                        int32_t *__restrict__ pivg, double *__restrict__ hinvg) {
-  __shared__ double cn[SVD_TALL_MAX_N];
-  __shared__ double2 rdiag[SVD_TALL_MAX_N];
-  __shared__ int pv[SVD_TALL_MAX_N];
+                                                        int32_t *__restrict__ pivg, double *__restrict__ hinvg,
+                                                        int maxN, int64_t slot) {
+  __shared__ double cn[SVD_QR_MAX_N];
+  __shared__ double2 rdiag[SVD_QR_MAX_N];
+  __shared__ int pv[SVD_QR_MAX_N];
   __shared__ int qsel;
   __shared__ double qnorm;
   const int t = blockIdx.x, b = idx[t];
@@ -1268,6 +1409,24 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   double2 *s = S + aOff[b];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   constexpr int NW = SVD_TALL_T / 64;
+  {
+    __shared__ double2 vbuf[513]; /* the reflector and its scale */
+    double2 *rg = RG + (int64_t)t * slot;
+    int32_t *piv = pivg + (int64_t)t * maxN;
+    double *hinv = hinvg + (int64_t)t * maxN;
+#define QR_REGS(R, C) qr_regs<R, C>(a, s, m, n, rg, piv, hinv, cn, pv, vbuf)
+    /* 64 of a thread's 128 registers hold the matrix; 80 or 96 spill */
+    if (m <= 256 && n <= 64) {
+      if (n <= 32) QR_REGS(4, 2);
+      else QR_REGS(4, 4);
+      return;
+    }
+    if (m <= 512 && n <= 32) {
+      QR_REGS(8, 2);
+      return;
+    }
+#undef QR_REGS
+  }
   for (int64_t e = tid; e < (int64_t)m * n; e += SVD_TALL_T) s[e] = a[e];
   for (int j = tid; j < n; j += SVD_TALL_T) pv[j] = j;
   __syncthreads();
@@ -1282,12 +1441,16 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   }
   __syncthreads();
   for (int j = 0; j < n; ++j) {
-    if (tid == 0) {
-      int best = j;
-      for (int c = j + 1; c < n; ++c)
-        if (cn[c] > cn[best]) best = c;
-      qsel = best;
-      qnorm = cn[best];
+    if (w == 0) { /* the largest remaining column, the first among equals */
+      double best = -1.0;
+      int bi = n;
+      for (int c = j + lane; c < n; c += 64)
+        if (cn[c] > best) { best = cn[c]; bi = c; }
+      wave_argmax(best, bi);
+      if (lane == 0) {
+        qsel = bi < n ? bi : j; /* no comparison holds: NaN */
+        qnorm = cn[bi < n ? bi : j];
+      }
     }
     __syncthreads();
     const int q = qsel;
@@ -1313,7 +1476,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;
     __syncthreads();
     if (tid == 0) {
-      hinvg[(int64_t)t * SVD_TALL_MAX_N + j] = sg > 0 ? 1.0 / (sg * (sg + ax0)) : 0.0;
+      hinvg[(int64_t)t * maxN + j] = sg > 0 ? 1.0 / (sg * (sg + ax0)) : 0.0;
       rdiag[j] = sg > 0 ? make_double2(-phx * sg, -phy * sg) : x0;
     }
     if (sg > 0) {
@@ -1333,7 +1496,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   }
   /* [R | I], row-major with leading dimension 2n + 1 */
   const int ld = tall_ld(n);
-  double2 *rg = RG + (int64_t)t * TALL_SLOT;
+  double2 *rg = RG + (int64_t)t * slot;
   for (int e = tid; e < n * 2 * n; e += SVD_TALL_T) {
     const int i = e / (2 * n), c = e - i * 2 * n;
     double2 v;
@@ -1341,30 +1504,138 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     else v = make_double2(c - n == i ? 1.0 : 0.0, 0.0);
     rg[i * ld + c] = v;
   }
-  for (int j = tid; j < n; j += SVD_TALL_T) pivg[(int64_t)t * SVD_TALL_MAX_N + j] = pv[j];
+  for (int j = tid; j < n; j += SVD_TALL_T) pivg[(int64_t)t * maxN + j] = pv[j];
 }
 
-__global__ __launch_bounds__(64) void k_tall_jacobi(const int32_t *__restrict__ idx, const int32_t *__restrict__ nn,
-                                                    double2 *__restrict__ RG) {
+template <int T>
+__global__ __launch_bounds__(T) void k_tall_jacobi(const int32_t *__restrict__ idx, const int32_t *__restrict__ nn,
+                                                   double2 *__restrict__ RG, int64_t slot) {
   extern __shared__ double2 lds[];
   const int t = blockIdx.x, n = nn[idx[t]], ld = tall_ld(n);
-  double2 *rg = RG + (int64_t)t * TALL_SLOT;
-  for (int e = threadIdx.x; e < n * ld; e += 64) lds[e] = rg[e];
+  double2 *rg = RG + (int64_t)t * slot;
+  double *red = (double *)(lds + n * ld);
+  for (int e = threadIdx.x; e < n * ld; e += T) lds[e] = rg[e];
   __syncthreads();
   const int npairs = (n + (n & 1)) / 2;
   int Lp = 64;
-  while (Lp > 1 && Lp * npairs > 64) Lp >>= 1;
+  while (Lp > 1 && Lp * npairs > T) Lp >>= 1;
   switch (Lp) {
-    case 8: jacobi_rows<8, 64>(lds, n, 2 * n, ld, nullptr); break;
-    case 4: jacobi_rows<4, 64>(lds, n, 2 * n, ld, nullptr); break;
-    case 2: jacobi_rows<2, 64>(lds, n, 2 * n, ld, nullptr); break;
-    case 1: jacobi_rows<1, 64>(lds, n, 2 * n, ld, nullptr); break;
-    case 16: jacobi_rows<16, 64>(lds, n, 2 * n, ld, nullptr); break;
-    case 32: jacobi_rows<32, 64>(lds, n, 2 * n, ld, nullptr); break;
-    default: jacobi_rows<64, 64>(lds, n, 2 * n, ld, nullptr); break;
+    case 64: jacobi_rows<64, T, true>(lds, n, 2 * n, ld, red); break;
+    case 32: jacobi_rows<32, T, true>(lds, n, 2 * n, ld, red); break;
+    default: jacobi_rows<16, T, true>(lds, n, 2 * n, ld, red); break;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < n * ld; e += 64) rg[e] = lds[e];
+  for (int e = threadIdx.x; e < n * ld; e += T) rg[e] = lds[e];
+}
+
+/* One round of a sweep of the row Jacobi over blocks of SVD_BLK rows of
+ * [R | I] (global memory), for matrices too wide for one CU's LDS: the
+ * blocks meet in round-robin pairs, workgroup (p, b) brings pair p of matrix
+ * b into LDS and rotates every row of one block against every row of the
+ * other, a wave per pair of rows; the first round also rotates the pairs
+ * inside each block.  A round is bound by the LDS traffic of its 8 (15)
+ * steps; one launch a round replaces one launch a step. */
+#define SVD_BLK 8
+#define SVD_BLK_T (64 * SVD_BLK)
+__host__ __device__ __forceinline__ size_t svd_block_lds(int n) { return (size_t)2 * SVD_BLK * tall_ld(n) * 16; }
+__global__ __launch_bounds__(SVD_BLK_T) void k_svd_block(const int32_t *__restrict__ idx, const int32_t *__restrict__ nn,
+                                                         double2 *__restrict__ RG, int64_t slot, int round,
+                                                         const int32_t *__restrict__ active, int32_t *__restrict__ rot) {
+  extern __shared__ double2 lds[];
+  const int t = blockIdx.y;
+  if (!active[t]) return;
+  const int n = nn[idx[t]], ld = tall_ld(n), W = 2 * n;
+  const int nb = (n + SVD_BLK - 1) / SVD_BLK, P = nb + (nb & 1), pr = blockIdx.x;
+  if (round >= P - 1 || pr >= P / 2) return;
+  const int p0 = rr_row(pr, round, P), p1 = rr_row(P - 1 - pr, round, P);
+  const int bi = min(p0, p1), bj = max(p0, p1); /* bj == nb: bi has no partner this round */
+  const int ci = min(SVD_BLK, n - bi * SVD_BLK), cj = bj < nb ? min(SVD_BLK, n - bj * SVD_BLK) : 0;
+  double2 *gi = RG + (int64_t)t * slot + (int64_t)bi * SVD_BLK * ld, *gj = RG + (int64_t)t * slot + (int64_t)bj * SVD_BLK * ld;
+  double2 *li = lds, *lj = lds + SVD_BLK * ld;
+  for (int e = threadIdx.x; e < ci * ld; e += SVD_BLK_T) li[e] = gi[e];
+  for (int e = threadIdx.x; e < cj * ld; e += SVD_BLK_T) lj[e] = gj[e];
+  __syncthreads();
+  const int g = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double eps = 2.220446049250313e-16;
+  const double thr = 4.0 * eps * sqrt((double)n), thr2 = thr * thr;
+  int rotated = 0;
+  const int inner = round == 0 ? SVD_BLK - 1 : 0;
+  for (int step = 0; step < inner + SVD_BLK; ++step) {
+    double2 *ri, *rj;
+    bool valid;
+    if (step < inner) { /* pairs inside a block: waves 0-3 block i, 4-7 block j */
+      const int h = g & 3, a = rr_row_fast(h, step, SVD_BLK), b = rr_row_fast(SVD_BLK - 1 - h, step, SVD_BLK);
+      const int c = g < 4 ? ci : cj;
+      double2 *l = g < 4 ? li : lj;
+      ri = l + min(a, b) * ld;
+      rj = l + max(a, b) * ld;
+      valid = max(a, b) < c;
+    } else {
+      const int b = (g + step - inner) & (SVD_BLK - 1);
+      ri = li + g * ld;
+      rj = lj + b * ld;
+      valid = g < ci && b < cj;
+    }
+    if (valid) { /* uniform over the wave */
+      double al = 0, be = 0, gx = 0, gy = 0;
+      for (int c = lane; c < n; c += 64) {
+        const double2 x = ri[c], y = rj[c];
+        al = fma(x.x, x.x, fma(x.y, x.y, al));
+        be = fma(y.x, y.x, fma(y.y, y.y, be));
+        gx = fma(x.x, y.x, fma(x.y, y.y, gx)); /* x conj(y) */
+        gy = fma(x.y, y.x, fma(-x.x, y.y, gy));
+      }
+      al = group_sum(al, 64);
+      be = group_sum(be, 64);
+      gx = group_sum(gx, 64);
+      gy = group_sum(gy, 64);
+      const double ag2 = gx * gx + gy * gy;
+      if (ag2 > 1e-290 && ag2 > thr2 * al * be) { /* the rotation of jacobi_rows */
+        rotated = 1;
+        const double rg = rsqrt_nr(ag2);
+        const double ex = gx * rg, ey = gy * rg;
+        const double zeta = (be - al) * (0.5 * rg), az = fabs(zeta);
+        double tn = az > 1e150 ? 0.5 / zeta : (zeta >= 0 ? 1.0 : -1.0) / (az + sqrt(fma(zeta, zeta, 1.0)));
+        const double cs = rsqrt_nr(fma(tn, tn, 1.0)), sn = cs * tn;
+        const double sx = sn * ex, sy = sn * ey, cx = cs * ex, cy = cs * ey;
+        for (int c = lane; c < W; c += 64) {
+          const double2 x = ri[c], y = rj[c];
+          ri[c] = make_double2(fma(cs, x.x, -fma(sx, y.x, -sy * y.y)), fma(cs, x.y, -fma(sx, y.y, sy * y.x)));
+          rj[c] = make_double2(fma(sn, x.x, fma(cx, y.x, -cy * y.y)), fma(sn, x.y, fma(cx, y.y, cy * y.x)));
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (rotated && lane == 0) rot[t] = 1;
+  for (int e = threadIdx.x; e < ci * ld; e += SVD_BLK_T) gi[e] = li[e];
+  for (int e = threadIdx.x; e < cj * ld; e += SVD_BLK_T) gj[e] = lj[e];
+}
+
+/* sigma and V of matrix t from [R' | G], a workgroup's threads over both.
+ * A row that is exactly zero gets the unit vector of its pivot: the pivoted
+ * QR leaves such rows last, for columns outside the others' span. */
+__device__ __forceinline__ void tall_sigma_v(const double2 *__restrict__ rg, int n, int ld, const int32_t *__restrict__ pv,
+                                             double *__restrict__ sgm, double *__restrict__ sig,
+                                             double2 *__restrict__ vo) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  for (int i = w; i < n; i += SVD_TALL_T / 64) {
+    double q = 0;
+    for (int c = lane; c < n; c += 64) q = fma(rg[i * ld + c].x, rg[i * ld + c].x, fma(rg[i * ld + c].y, rg[i * ld + c].y, q));
+    q = group_sum(q, 64);
+    if (lane == 0) {
+      sgm[i] = sqrt(q);
+      sig[i] = sqrt(q);
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < n * n; e += SVD_TALL_T) { /* V column i = P conj(row i of R') / sigma_i */
+    const int i = e / n, j = e - i * n;
+    const double inv = sgm[i] > 0 ? 1.0 / sgm[i] : 0.0;
+    const double2 r = rg[i * ld + j];
+    vo[(int64_t)i * n + pv[j]] =
+        sgm[i] > 0 ? make_double2(r.x * inv, -r.y * inv) : make_double2(sgm[i] == 0 && i == j ? 1.0 : 0.0, 0.0);
+  }
 }
 
 __global__ __launch_bounds__(SVD_TALL_T) void k_tall_w(const int32_t *__restrict__ idx,
@@ -1374,35 +1645,19 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_w(const int32_t *__restrict
                                                        const double2 *__restrict__ RG, const int32_t *__restrict__ pivg,
                                                        const double *__restrict__ hinvg,
                                                        const int64_t *__restrict__ vOff, double2 *__restrict__ Vout,
-                                                       const int64_t *__restrict__ sOff, double *__restrict__ sig) {
+                                                       const int64_t *__restrict__ sOff, double *__restrict__ sig,
+                                                       int maxN, int64_t slot) {
   __shared__ double sgm[SVD_TALL_MAX_N];
   extern __shared__ double2 lds[]; /* 2 n^2: T^{-1} and Z */
   const int t = blockIdx.x, b = idx[t];
   const int m = mm[b], n = nn[b], ld = tall_ld(n);
   double2 *a = A + aOff[b];
-  const double2 *s = S + aOff[b], *rg = RG + (int64_t)t * TALL_SLOT;
-  const int32_t *pv = pivg + (int64_t)t * SVD_TALL_MAX_N;
-  const double *hinv = hinvg + (int64_t)t * SVD_TALL_MAX_N;
+  const double2 *s = S + aOff[b], *rg = RG + (int64_t)t * slot;
+  const int32_t *pv = pivg + (int64_t)t * maxN;
+  const double *hinv = hinvg + (int64_t)t * maxN;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   constexpr int NW = SVD_TALL_T / 64;
-  for (int i = w; i < n; i += NW) {
-    double q = 0;
-    for (int c = lane; c < n; c += 64) q = fma(rg[i * ld + c].x, rg[i * ld + c].x, fma(rg[i * ld + c].y, rg[i * ld + c].y, q));
-    q = group_sum(q, 64);
-    if (lane == 0) {
-      sgm[i] = sqrt(q);
-      sig[sOff[b] + i] = sqrt(q);
-    }
-  }
-  __syncthreads();
-  /* V column i = P conj(row i of R') / sigma_i */
-  double2 *vo = Vout + vOff[b];
-  for (int e = tid; e < n * n; e += SVD_TALL_T) {
-    const int i = e / n, j = e - i * n;
-    const double inv = sgm[i] > 0 ? 1.0 / sgm[i] : 0.0;
-    const double2 r = rg[i * ld + j];
-    vo[(int64_t)i * n + pv[j]] = make_double2(r.x * inv, -r.y * inv);
-  }
+  tall_sigma_v(rg, n, ld, pv, sgm, sig + sOff[b], Vout + vOff[b]);
   /* W = Q X, X = [sigma_c conj(G[c, :])^T; 0] (m x n, zero below row n),
    * Q = H_0 ... H_{n-1}, H_j = I - tau_j v_j v_j^H, v_j = column j of S on
    * rows >= j, tau_j = hinv[j] (0: no reflector).  Compact WY form:
@@ -1513,6 +1768,41 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_w(const int32_t *__restrict
     }
   }
 #undef TALL_X
+}
+
+/* the same for the matrices of k_svd_block, whose T and Z' do not fit in LDS:
+ * sigma and V by the first workgroup of a matrix, then a wave per column of
+ * X applies the reflectors to it, last first */
+__global__ __launch_bounds__(SVD_TALL_T) void k_wide_w(const int32_t *__restrict__ idx,
+                                                       const int64_t *__restrict__ aOff,
+                                                       const int32_t *__restrict__ mm, const int32_t *__restrict__ nn,
+                                                       double2 *__restrict__ A, const double2 *__restrict__ S,
+                                                       const double2 *__restrict__ RG, const int32_t *__restrict__ pivg,
+                                                       const double *__restrict__ hinvg,
+                                                       const int64_t *__restrict__ vOff, double2 *__restrict__ Vout,
+                                                       const int64_t *__restrict__ sOff, double *__restrict__ sig,
+                                                       int maxN, int64_t slot) {
+  __shared__ double sgm[SVD_QR_MAX_N];
+  const int t = blockIdx.y, b = idx[t];
+  const int m = mm[b], n = nn[b], ld = tall_ld(n);
+  const double2 *s = S + aOff[b], *rg = RG + (int64_t)t * slot;
+  const double *hinv = hinvg + (int64_t)t * maxN;
+  if (blockIdx.x == 0) {
+    tall_sigma_v(rg, n, ld, pivg + (int64_t)t * maxN, sgm, sig + sOff[b], Vout + vOff[b]);
+    return; /* the whole workgroup */
+  }
+  const int lane = threadIdx.x & 63, c = (int)(blockIdx.x - 1) * (SVD_TALL_T / 64) + (int)(threadIdx.x >> 6);
+  if (c >= n) return;
+  double q = 0;
+  for (int j = lane; j < n; j += 64) q = fma(rg[c * ld + j].x, rg[c * ld + j].x, fma(rg[c * ld + j].y, rg[c * ld + j].y, q));
+  const double sg = sqrt(group_sum(q, 64));
+  double2 *y = A + aOff[b] + (int64_t)c * m;
+  for (int r = lane; r < m; r += 64)
+    y[r] = r < n ? make_double2(sg * rg[c * ld + n + r].x, -sg * rg[c * ld + n + r].y) : make_double2(0, 0);
+  for (int j = n - 1; j >= 0; --j) {
+    __threadfence_block(); /* every lane reads rows that others wrote */
+    if (hinv[j] != 0) house_apply_wave(s + (int64_t)j * m, y, j, m, hinv[j], lane);
+  }
 }
 
 /* ---------------------------------------------------- orthogonalization */
@@ -2104,8 +2394,11 @@ int bfk_init(void) {
   /* k_tall_w also holds sigma in static LDS (SVD_TALL_MAX_N doubles) */
   g_tallOk = g_ldsCap >= svd_tall_lds(SVD_TALL_MAX_N) &&
              g_ldsCap >= svd_tall_w_lds(SVD_TALL_MAX_N) + SVD_TALL_MAX_N * 8 &&
-             hipFuncSetAttribute((const void *)k_tall_jacobi, hipFuncAttributeMaxDynamicSharedMemorySize,
+             g_ldsCap >= svd_block_lds(SVD_QR_MAX_N) &&
+             hipFuncSetAttribute((const void *)k_tall_jacobi<SVD_TALL_T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)svd_tall_lds(SVD_TALL_MAX_N)) == hipSuccess &&
+             hipFuncSetAttribute((const void *)k_svd_block, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)svd_block_lds(SVD_QR_MAX_N)) == hipSuccess &&
              hipFuncSetAttribute((const void *)k_tall_w, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)svd_tall_w_lds(SVD_TALL_MAX_N)) == hipSuccess;
   if (!g_tallOk) (void)hipGetLastError();
@@ -2203,6 +2496,19 @@ static void release(void *p) {
 
 void bfk_free(void *p) {
   if (p) release(p);
+}
+
+void *bfk_host_malloc(size_t bytes) {
+  void *p = nullptr;
+  if (bfk_init() || hipHostMalloc(&p, bytes ? bytes : 16, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return p;
+}
+
+void bfk_host_free(void *p) {
+  if (p) (void)hipHostFree(p);
 }
 
 /* released at the next bfk_sync, after the work queued before it is done;
@@ -2549,19 +2855,17 @@ int bfk_convert(int64_t n, const void *src, void *dst, int to32) {
   return 0;
 }
 
-/* batched SVD: tables and matrices already in device memory */
-int bfk_svd_jacobi(int64_t batch, const int64_t *dAOff, const int32_t *dM, const int32_t *dN, double *dA,
-                   const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, int maxSweeps) {
+/* matrices idx[0 .. nb) of a batch, one workgroup each */
+int bfk_svd_jacobi(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,
+                   double *dA, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, int maxSweeps) {
   if (bfk_init()) return -1;
-  if (batch <= 0) return 0;
   const int64_t maxGrid = 1 << 30;
-  for (int64_t b0 = 0; b0 < batch; b0 += maxGrid) {
-    int64_t nb = batch - b0 < maxGrid ? batch - b0 : maxGrid;
-    hipLaunchKernelGGL(k_svd_jacobi, dim3((unsigned)nb), dim3(256), 0, g_stream, dAOff + b0, dM + b0, dN + b0,
-                       (double2 *)dA, dVOff + b0, (double2 *)dV, dSOff + b0, dSig, maxSweeps);
+  for (int64_t b0 = 0; b0 < nb; b0 += maxGrid) {
+    const int64_t n = nb - b0 < maxGrid ? nb - b0 : maxGrid;
+    hipLaunchKernelGGL(k_svd_jacobi, dim3((unsigned)n), dim3(256), 0, g_stream, dIdx + b0, dAOff, dM, dN,
+                       (double2 *)dA, dVOff, (double2 *)dV, dSOff, dSig, maxSweeps);
     BFK_CHECK(hipGetLastError());
   }
-  BFK_CHECK(hipStreamSynchronize(g_stream));
   return 0;
 }
 
@@ -2620,44 +2924,78 @@ int bfk_svd_jacobi_big(int64_t nb, const int32_t *dBig, const int64_t *dAOff, co
 }
 
 int bfk_svd_tall_max_n(void) { return g_tallOk ? SVD_TALL_MAX_N : 0; }
+int bfk_svd_qr_max_n(void) { return g_tallOk ? SVD_QR_MAX_N : 0; }
 
-/* tall matrices idx[0 .. nb) of a batch (m >= 2n, n <= bfk_svd_tall_max_n()):
- * k_tall_qr, k_tall_jacobi, k_tall_w, one workgroup per matrix each; dS is
- * scratch of the size of dA; maxSweeps is not used (the row Jacobi stops by
- * its own test, at most 40 sweeps) */
-int bfk_svd_jacobi_tall(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,
-                        double *dA, double *dS, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig,
-                        int maxSweeps, int maxN) {
-  (void)maxSweeps;
+/* bytes of scratch beside the copy of the matrices: the triangles, the
+ * reflectors' scales and the pivots of nb matrices, and two flags each */
+size_t bfk_svd_qr_scratch(int64_t nb, int maxN) {
+  return (size_t)nb * ((size_t)tall_slot(maxN) * 16 + (size_t)maxN * 12 + 8);
+}
+
+/* Matrices idx[0 .. nb) of a batch (n <= maxN, m >= n), all of at most or all
+ * of more than SVD_TALL_MAX_N columns (and at most SVD_QR_MAX_N): the QR, the
+ * Jacobi on the triangles, then W; a workgroup per matrix each, or the block
+ * rounds for the wider ones.  dS is scratch of the size of dA, dWork of
+ * bfk_svd_qr_scratch bytes. */
+int bfk_svd_qr(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN, double *dA,
+               double *dS, const int64_t *dVOff, double *dV, const int64_t *dSOff, double *dSig, void *dWork,
+               int maxSweeps, int maxN) {
   if (bfk_init()) return -1;
   if (nb <= 0) return 0;
-  if (!g_tallOk || maxN > SVD_TALL_MAX_N || nb > (1 << 30)) return -3;
-  double2 *rg = nullptr;
-  int32_t *piv = nullptr;
-  double *hinv = nullptr;
-  BFK_CHECK(hipMalloc((void **)&rg, (size_t)nb * TALL_SLOT * 16));
-  BFK_CHECK(hipMalloc((void **)&piv, (size_t)nb * SVD_TALL_MAX_N * 4));
-  BFK_CHECK(hipMalloc((void **)&hinv, (size_t)nb * SVD_TALL_MAX_N * 8));
-  int rc = 0;
+  if (!g_tallOk || maxN > SVD_QR_MAX_N || nb > 65535) return -3;
+  const int64_t slot = tall_slot(maxN);
+  double2 *rg = (double2 *)dWork;
+  double *hinv = (double *)(rg + nb * slot);
+  int32_t *piv = (int32_t *)(hinv + nb * maxN), *dAct = piv + nb * maxN, *dRot = dAct + nb;
   hipLaunchKernelGGL(k_tall_qr, dim3((unsigned)nb), dim3(SVD_TALL_T), 0, g_stream, dIdx, dAOff, dM, dN,
-                     (const double2 *)dA, (double2 *)dS, rg, piv, hinv);
-  if (hipGetLastError() != hipSuccess) rc = -1;
-  if (!rc) {
-    hipLaunchKernelGGL(k_tall_jacobi, dim3((unsigned)nb), dim3(64), svd_tall_lds(maxN), g_stream, dIdx, dN, rg);
-    if (hipGetLastError() != hipSuccess) rc = -1;
+                     (const double2 *)dA, (double2 *)dS, rg, piv, hinv, maxN, slot);
+  BFK_CHECK(hipGetLastError());
+  if (maxN <= SVD_TALL_MAX_N) {
+    /* 8 pairs of 32 lanes fill 4 waves; wider ones take 16 */
+    if (maxN <= 16)
+      hipLaunchKernelGGL(k_tall_jacobi<256>, dim3((unsigned)nb), dim3(256), svd_tall_lds(maxN), g_stream, dIdx, dN, rg,
+                         slot);
+    else
+      hipLaunchKernelGGL(k_tall_jacobi<SVD_TALL_T>, dim3((unsigned)nb), dim3(SVD_TALL_T), svd_tall_lds(maxN), g_stream,
+                         dIdx, dN, rg, slot);
+    BFK_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(k_tall_w, dim3((unsigned)nb), dim3(SVD_TALL_T), svd_tall_w_lds(maxN), g_stream, dIdx, dAOff, dM,
+                       dN, (double2 *)dA, (const double2 *)dS, (const double2 *)rg, piv, hinv, dVOff, (double2 *)dV,
+                       dSOff, dSig, maxN, slot);
+    BFK_CHECK(hipGetLastError());
+    return 0;
   }
-  if (!rc) {
-    hipLaunchKernelGGL(k_tall_w, dim3((unsigned)nb), dim3(SVD_TALL_T), svd_tall_w_lds(maxN), g_stream, dIdx, dAOff,
-                       dM, dN,
-                       (double2 *)dA, (const double2 *)dS, (const double2 *)rg, piv, hinv, dVOff, (double2 *)dV, dSOff,
-                       dSig);
-    if (hipGetLastError() != hipSuccess) rc = -1;
+  const int blocks = (maxN + SVD_BLK - 1) / SVD_BLK, P = blocks + (blocks & 1);
+  int32_t *act = (int32_t *)malloc((size_t)nb * 8), *rot = act + nb;
+  if (!act) return -2;
+  for (int64_t i = 0; i < nb; ++i) act[i] = 1;
+  hipError_t e = hipSuccess;
+  for (int sweep = 0; sweep < maxSweeps && e == hipSuccess; ++sweep) {
+    int any = 0;
+    for (int64_t i = 0; i < nb; ++i) {
+      any |= act[i];
+      rot[i] = 0;
+    }
+    if (!any) break;
+    e = hipMemcpyAsync(dAct, act, (size_t)nb * 8, hipMemcpyHostToDevice, g_stream); /* the flags, rot cleared */
+    for (int round = 0; round < P - 1 && e == hipSuccess; ++round) {
+      hipLaunchKernelGGL(k_svd_block, dim3((unsigned)(P / 2), (unsigned)nb), dim3(SVD_BLK_T), svd_block_lds(maxN),
+                         g_stream, dIdx, dN, rg, slot, round, dAct, dRot);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(rot, dRot, (size_t)nb * 4, hipMemcpyDeviceToHost, g_stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(g_stream);
+    for (int64_t i = 0; i < nb; ++i) act[i] = act[i] && rot[i];
   }
-  if (hipStreamSynchronize(g_stream) != hipSuccess) rc = -1;
-  (void)hipFree(rg);
-  (void)hipFree(piv);
-  (void)hipFree(hinv);
-  return rc;
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_wide_w, dim3((unsigned)(1 + (maxN + SVD_TALL_T / 64 - 1) / (SVD_TALL_T / 64)), (unsigned)nb),
+                       dim3(SVD_TALL_T), 0, g_stream, dIdx, dAOff, dM, dN, (double2 *)dA, (const double2 *)dS,
+                       (const double2 *)rg, piv, hinv, dVOff, (double2 *)dV, dSOff, dSig, maxN, slot);
+    e = hipGetLastError();
+  }
+  free(act);
+  BFK_CHECK(e);
+  return 0;
 }
 
 size_t bfk_ortho_units(int rows, int n) { return ortho_units(rows, n); }

@@ -192,82 +192,146 @@ static int cmp_sig_desc(const void *a, const void *b) {
 /* the largest smaller side of a matrix the batched SVD takes (its cost
  * grows as the square of the column count) */
 #define SVD_MAX_COLS 1024
-/* matrices of at least this many entries get the whole chip per SVD */
-#define SVD_BIG_ENTRIES (1 << 15)
+/* The workspace of a streamer's SVDs: device memory and page-locked host
+ * memory for the copies, grown as needed and released with the streamer
+ * (bounded by what its largest round takes).  A call without one makes its
+ * own, in ordinary host memory. */
+typedef struct {
+  char *dev, *host;
+  size_t devBytes, hostBytes;
+  int locked; /* host is page-locked */
+} SvdWork;
 
-/* One-sided Jacobi SVDs of a batch whose tables (host copies h*, device
- * copies d*) are in place: large matrices take the per-step launches over
- * the whole chip, the rest one workgroup each in one launch.  The device
- * tables are overwritten (with the small matrices' entries). */
-static int jacobi_dispatch(int64_t nj, const int64_t *aOff, const int32_t *M, const int32_t *N, const int64_t *vOff,
-                           const int64_t *sOff, void *dAo, void *dM, void *dN, void *dVo, void *dSo, void *dA,
-                           void *dV, void *dS) {
-  int32_t *bigIdx = malloc(nz(nj) * sizeof(int32_t)), *tallIdx = malloc(nz(nj) * sizeof(int32_t));
-  int64_t *sA = malloc(nz(nj) * 8), *sV = malloc(nz(nj) * 8), *sS = malloc(nz(nj) * 8);
-  int32_t *sM = malloc(nz(nj) * 4), *sN = malloc(nz(nj) * 4);
-  int64_t nbig = 0, nsmall = 0, ntall = 0, tallEnd = 0;
-  int maxN = 0, maxTallN = 0, rc = 0;
-  const int tallMax = bfk_svd_tall_max_n();
+static void svd_host_free(SvdWork *w) {
+  if (w->locked) bfk_host_free(w->host);
+  else free(w->host);
+  w->host = NULL;
+  w->hostBytes = 0;
+}
+
+static int svd_work(SvdWork *w, size_t dev, size_t host) {
+  if (dev > w->devBytes) {
+    bfk_free(w->dev);
+    w->devBytes = 0;
+    w->dev = bfk_malloc(dev + dev / 4);
+    if (!w->dev) return -2;
+    w->devBytes = dev + dev / 4;
+  }
+  if (host > w->hostBytes) {
+    svd_host_free(w);
+    w->host = w->locked ? bfk_host_malloc(host + host / 4) : malloc(host);
+    if (!w->host) return -2;
+    w->hostBytes = w->locked ? host + host / 4 : host;
+  }
+  return 0;
+}
+
+static void svd_work_free(SvdWork *w) {
+  bfk_free(w->dev);
+  svd_host_free(w);
+  w->dev = NULL;
+  w->devBytes = 0;
+}
+
+/* How a batch of one-sided Jacobi SVDs is split over the paths.  A matrix
+ * of n columns and m >= n rows goes
+ *   0, 1  through its QR and the Jacobi of the triangle: in one CU's LDS up
+ *         to 70 columns, by blocks of rows up to 256.  256 x 60: 0.9 ms
+ *         where the column Jacobi took 12; 384 x 128: 3 ms where a launch
+ *         per step took 14;
+ *   2     beyond 256 columns, over the whole chip a step per launch: the
+ *         one-workgroup QR would cost what the narrower Jacobi saves;
+ *   3     with more than 256 rows and less than 2^15 entries, one workgroup
+ *         on the columns as they are (k_svd_jacobi says why these stay). */
+typedef struct {
+  int32_t *idx; /* four lists of nj */
+  int64_t cnt[4], chunk[4];
+  int maxN[4];
+  int64_t end;    /* entries of A that the QR copies */
+  size_t scratch; /* bytes of one launch sequence of a QR path */
+  size_t bytes;   /* device bytes of it all */
+} SvdSplit;
+
+/* most scratch of one launch sequence of the QR paths */
+#define SVD_SCRATCH_MAX ((size_t)1 << 30)
+#define SVD_QR_ROWS 256
+#define SVD_QR_ENTRIES (1 << 15)
+
+static int svd_split(SvdSplit *p, int64_t nj, const int64_t *aOff, const int32_t *M, const int32_t *N) {
+  memset(p, 0, sizeof(*p));
+  p->idx = malloc(nz(4 * nj) * sizeof(int32_t));
+  if (!p->idx) return -2;
+  const int limit[2] = {bfk_svd_tall_max_n(), bfk_svd_qr_max_n()};
   for (int64_t i = 0; i < nj; ++i) {
-    if ((int64_t)M[i] * N[i] >= SVD_BIG_ENTRIES && N[i] >= 2 && N[i] <= tallMax && M[i] >= 2 * N[i]) {
-      /* tall: QR first, the Jacobi on the n x n triangle in LDS */
-      tallIdx[ntall++] = (int32_t)i;
-      if (N[i] > maxTallN) maxTallN = N[i];
-      if (aOff[i] + (int64_t)M[i] * N[i] > tallEnd) tallEnd = aOff[i] + (int64_t)M[i] * N[i];
-    } else if ((int64_t)M[i] * N[i] >= SVD_BIG_ENTRIES && N[i] >= 2) {
-      bigIdx[nbig++] = (int32_t)i;
-      if (N[i] > maxN) maxN = N[i];
-    } else {
-      sA[nsmall] = aOff[i];
-      sV[nsmall] = vOff[i];
-      sS[nsmall] = sOff[i];
-      sM[nsmall] = M[i];
-      sN[nsmall] = N[i];
-      ++nsmall;
+    if (N[i] < 1) continue;
+    const int64_t e = (int64_t)M[i] * N[i];
+    const int c = M[i] > SVD_QR_ROWS && e < SVD_QR_ENTRIES ? 3 : N[i] <= limit[0] ? 0 : N[i] <= limit[1] ? 1 : 2;
+    p->idx[c * nj + p->cnt[c]++] = (int32_t)i;
+    if (N[i] > p->maxN[c]) p->maxN[c] = N[i];
+    if (c < 2 && aOff[i] + e > p->end) p->end = aOff[i] + e;
+  }
+  for (int c = 0; c < 4; ++c) p->chunk[c] = p->cnt[c] > 0 ? p->cnt[c] : 1;
+  for (int c = 0; c < 2; ++c) {
+    if (!p->cnt[c]) continue;
+    const int64_t most = (int64_t)(SVD_SCRATCH_MAX / bfk_svd_qr_scratch(1, p->maxN[c]));
+    if (p->chunk[c] > most) p->chunk[c] = most;
+    if (p->chunk[c] > 65535) p->chunk[c] = 65535;
+    const size_t b = bfk_svd_qr_scratch(p->chunk[c], p->maxN[c]);
+    if (b > p->scratch) p->scratch = b;
+  }
+  p->scratch = (p->scratch + 15) & ~(size_t)15;
+  p->bytes = (size_t)p->end * 16 + p->scratch;
+  return 0;
+}
+
+/* The SVDs, with the tables (and the split's lists, at dIdx) in device
+ * memory; w has the split's bytes.  Returns with the work queued. */
+static int svd_run(const SvdSplit *p, int64_t nj, const int32_t *dIdx, char *w, void *dAo, void *dM, void *dN, void *dVo,
+                   void *dSo, void *dA, void *dV, void *dS) {
+  int rc = 0;
+  for (int c = 0; c < 4; ++c)
+    for (int64_t i = 0; i < p->cnt[c] && !rc; i += p->chunk[c]) {
+      const int32_t *ix = dIdx + c * nj + i;
+      const int64_t n = p->cnt[c] - i < p->chunk[c] ? p->cnt[c] - i : p->chunk[c];
+      if (c < 2)
+        rc = bfk_svd_qr(n, ix, dAo, dM, dN, dA, (double *)w, dVo, dV, dSo, dS, w + (size_t)p->end * 16, 60, p->maxN[c]);
+      else if (c == 2)
+        rc = bfk_svd_jacobi_big(n, ix, dAo, dM, dN, dA, dVo, dV, dSo, dS, 60, p->maxN[c]);
+      else
+        rc = bfk_svd_jacobi(n, ix, dAo, dM, dN, dA, dVo, dV, dSo, dS, 60);
     }
-  }
-  if (ntall) {
-    void *dT = bfk_malloc((size_t)ntall * 4), *dScr = bfk_malloc((size_t)tallEnd * 16);
-    if (!dT || !dScr) rc = -2;
-    if (!rc) rc = bfk_h2d(dT, tallIdx, (size_t)ntall * 4);
-    if (!rc) rc = bfk_svd_jacobi_tall(ntall, dT, dAo, dM, dN, dA, dScr, dVo, dV, dSo, dS, 60, maxTallN);
-    bfk_free(dT);
-    bfk_free(dScr);
-  }
-  if (nbig && !rc) {
-    void *dB = bfk_malloc((size_t)nbig * 4);
-    if (!dB) rc = -2;
-    if (!rc) rc = bfk_h2d(dB, bigIdx, (size_t)nbig * 4);
-    if (!rc) rc = bfk_svd_jacobi_big(nbig, dB, dAo, dM, dN, dA, dVo, dV, dSo, dS, 60, maxN);
-    bfk_free(dB);
-  }
-  if ((nbig || ntall) && !rc) {
-    if (nsmall) { /* the small ones' tables */
-      rc = bfk_h2d(dAo, sA, (size_t)nsmall * 8);
-      if (!rc) rc = bfk_h2d(dVo, sV, (size_t)nsmall * 8);
-      if (!rc) rc = bfk_h2d(dSo, sS, (size_t)nsmall * 8);
-      if (!rc) rc = bfk_h2d(dM, sM, (size_t)nsmall * 4);
-      if (!rc) rc = bfk_h2d(dN, sN, (size_t)nsmall * 4);
-    }
-  }
-  if (!rc && nsmall) rc = bfk_svd_jacobi(nsmall, dAo, dM, dN, dA, dVo, dV, dSo, dS, 60);
-  free(bigIdx); free(tallIdx); free(sA); free(sV); free(sS); free(sM); free(sN);
   return rc;
 }
 
-/* All jobs in one launch.  Wide blocks (m < n) are decomposed through
- * their conjugate transpose so the kernel always sees n <= m columns. */
-static int svd_batch(SvdJob *jobs, size_t nj, double tol) {
+/* one batch whose tables are in place (host and device copies) */
+static int jacobi_dispatch(int64_t nj, const int64_t *aOff, const int32_t *M, const int32_t *N, void *dAo, void *dM,
+                           void *dN, void *dVo, void *dSo, void *dA, void *dV, void *dS) {
+  SvdSplit p;
+  int rc = svd_split(&p, nj, aOff, M, N);
+  if (rc) return rc;
+  char *w = bfk_malloc(p.bytes + (size_t)(4 * nj) * 4 + 16);
+  rc = w ? bfk_h2d(w + p.bytes, p.idx, (size_t)(4 * nj) * 4) : -2;
+  if (!rc) rc = svd_run(&p, nj, (const int32_t *)(w + p.bytes), w, dAo, dM, dN, dVo, dSo, dA, dV, dS);
+  const int rs = bfk_sync();
+  bfk_free(w);
+  free(p.idx);
+  return rc ? rc : rs;
+}
+
+/* All jobs together.  Wide blocks (m < n) are decomposed through their
+ * conjugate transpose so the kernels always see n <= m columns.  One copy
+ * takes the tables and the matrices to the device, one brings W, V and the
+ * singular values back. */
+static int svd_batch(SvdJob *jobs, size_t nj, double tol, SvdWork *work) {
   if (nj == 0) return 0;
-  int64_t *aOff = malloc(nj * sizeof(int64_t)), *vOff = malloc(nj * sizeof(int64_t)),
-          *sOff = malloc(nj * sizeof(int64_t));
-  int32_t *M = malloc(nj * sizeof(int32_t)), *N = malloc(nj * sizeof(int32_t));
+  int64_t *aOff = malloc(3 * nj * sizeof(int64_t)), *vOff = aOff + nj, *sOff = vOff + nj;
+  int32_t *M = malloc(2 * nj * sizeof(int32_t)), *N = M + nj;
   int64_t totA = 0, totV = 0, totS = 0;
   for (size_t i = 0; i < nj; ++i) {
     int wide = jobs[i].m < jobs[i].n;
     int64_t m = wide ? jobs[i].n : jobs[i].m, n = wide ? jobs[i].m : jobs[i].n;
     if (n > SVD_MAX_COLS) {
-      free(aOff); free(vOff); free(sOff); free(M); free(N);
+      free(aOff); free(M);
       return -3;
     }
     M[i] = (int32_t)m;
@@ -279,9 +343,27 @@ static int svd_batch(SvdJob *jobs, size_t nj, double tol) {
     totV += n * n;
     totS += n;
   }
-  BfComplex *hA = malloc((size_t)(totA ? totA : 1) * sizeof(BfComplex));
-  BfComplex *hV = malloc((size_t)(totV ? totV : 1) * sizeof(BfComplex));
-  double *hS = malloc((size_t)(totS ? totS : 1) * sizeof(double));
+  SvdSplit p;
+  int rc = svd_split(&p, (int64_t)nj, aOff, M, N);
+  /* device: [offsets, sizes, lists | A | V | sigma | workspace]; the host
+   * copy holds the first four */
+  const size_t tabs = (nj * (3 * 8 + 2 * 4 + 4 * 4) + 15) & ~(size_t)15;
+  const size_t offA = tabs, offV = offA + (size_t)totA * 16, offS = offV + (size_t)totV * 16;
+  const size_t offW = offS + (((size_t)totS * 8 + 15) & ~(size_t)15);
+  SvdWork own;
+  memset(&own, 0, sizeof(own));
+  SvdWork *wk = work ? work : &own;
+  if (!rc) rc = svd_work(wk, offW + p.bytes + 16, offW + 16);
+  if (rc) {
+    free(aOff); free(M); free(p.idx);
+    svd_work_free(&own);
+    return rc;
+  }
+  BfComplex *hA = (BfComplex *)(wk->host + offA), *hV = (BfComplex *)(wk->host + offV);
+  double *hS = (double *)(wk->host + offS);
+  memcpy(wk->host, aOff, 3 * nj * 8);
+  memcpy(wk->host + 3 * nj * 8, M, 2 * nj * 4);
+  memcpy(wk->host + 3 * nj * 8 + 2 * nj * 4, p.idx, 4 * nj * 4);
   for (size_t i = 0; i < nj; ++i) {
     SvdJob *J = &jobs[i];
     BfComplex *dst = hA + aOff[i];
@@ -292,29 +374,14 @@ static int svd_batch(SvdJob *jobs, size_t nj, double tol) {
       memcpy(dst, J->a, (size_t)(J->m * J->n) * sizeof(BfComplex));
     }
   }
-  int rc = 0;
-  void *dA = NULL, *dV = NULL, *dS = NULL, *dAo = NULL, *dVo = NULL, *dSo = NULL, *dM = NULL, *dN = NULL;
-  dA = bfk_malloc((size_t)(totA ? totA : 1) * 16);
-  dV = bfk_malloc((size_t)(totV ? totV : 1) * 16);
-  dS = bfk_malloc((size_t)(totS ? totS : 1) * 8);
-  dAo = bfk_malloc(nj * 8);
-  dVo = bfk_malloc(nj * 8);
-  dSo = bfk_malloc(nj * 8);
-  dM = bfk_malloc(nj * 4);
-  dN = bfk_malloc(nj * 4);
-  if (!dA || !dV || !dS || !dAo || !dVo || !dSo || !dM || !dN) rc = -2;
-  if (!rc) rc = bfk_h2d(dA, hA, (size_t)totA * 16);
-  if (!rc) rc = bfk_h2d(dAo, aOff, nj * 8);
-  if (!rc) rc = bfk_h2d(dVo, vOff, nj * 8);
-  if (!rc) rc = bfk_h2d(dSo, sOff, nj * 8);
-  if (!rc) rc = bfk_h2d(dM, M, nj * 4);
-  if (!rc) rc = bfk_h2d(dN, N, nj * 4);
-  if (!rc) rc = jacobi_dispatch((int64_t)nj, aOff, M, N, vOff, sOff, dAo, dM, dN, dVo, dSo, dA, dV, dS);
-  if (!rc) rc = bfk_d2h(hA, dA, (size_t)totA * 16);
-  if (!rc) rc = bfk_d2h(hV, dV, (size_t)totV * 16);
-  if (!rc) rc = bfk_d2h(hS, dS, (size_t)totS * 8);
-  bfk_free(dA); bfk_free(dV); bfk_free(dS); bfk_free(dAo); bfk_free(dVo); bfk_free(dSo);
-  bfk_free(dM); bfk_free(dN);
+  char *d = wk->dev;
+  int64_t *dAo = (int64_t *)d, *dVo = dAo + nj, *dSo = dVo + nj;
+  int32_t *dM = (int32_t *)(dSo + nj), *dN = dM + nj, *dIdx = dN + nj;
+  rc = bfk_h2d(d, wk->host, offV);
+  if (!rc) rc = svd_run(&p, (int64_t)nj, dIdx, d + offW, dAo, dM, dN, dVo, dSo, d + offA, d + offV, d + offS);
+  if (!rc) rc = bfk_d2h(wk->host + offA, d + offA, offS + (size_t)totS * 8 - offA);
+  if (rc) (void)bfk_sync();
+  free(p.idx);
   for (size_t i = 0; i < nj && !rc; ++i) {
     SvdJob *J = &jobs[i];
     const int64_t m = M[i], n = N[i];
@@ -348,7 +415,8 @@ static int svd_batch(SvdJob *jobs, size_t nj, double tol) {
     }
     free(si);
   }
-  free(hA); free(hV); free(hS); free(aOff); free(vOff); free(sOff); free(M); free(N);
+  free(aOff); free(M);
+  svd_work_free(&own);
   return rc;
 }
 
@@ -381,7 +449,7 @@ int bfhipSvdBatched(BfSize batch, BfSize const *m, BfSize const *n, BfComplex co
     jobs[i].a = cdup(A + off, jobs[i].m * jobs[i].n);
     off += jobs[i].m * jobs[i].n;
   }
-  int rc = svd_batch(jobs, batch, tol);
+  int rc = svd_batch(jobs, batch, tol, NULL);
   int64_t uo = 0, wo = 0;
   for (BfSize i = 0; i < batch; ++i) {
     if (!rc) {
@@ -417,7 +485,8 @@ typedef struct {
  * width did not saturate); a rejected sketch (fell[i] = 1) and every job
  * with width 0, width >= min(m, n) or width > SVD_MAX_COLS take the full SVD.  The
  * rule for k is svd_batch's (linalg.c:26-35). */
-static int svd_batch_sketch(SvdJob *jobs, size_t nj, double tol, const int64_t *width, uint64_t seed, int *fell) {
+static int svd_batch_sketch(SvdJob *jobs, size_t nj, double tol, const int64_t *width, uint64_t seed, int *fell,
+                            SvdWork *work) {
   if (nj == 0) return 0;
   if (bfk_sketch_jobs_bytes() != (int)sizeof(SketchJob)) return -1;
   size_t *sk = malloc(nz((int64_t)nj) * sizeof(size_t)), *full = malloc(nz((int64_t)nj) * sizeof(size_t));
@@ -487,13 +556,9 @@ static int svd_batch_sketch(SvdJob *jobs, size_t nj, double tol, const int64_t *
     if (!rc) rc = bfk_h2d(dN, N, ns * 4);
     if (!rc) rc = bfk_h2d(dW, Wd, ns * 4);
     if (!rc) rc = bfk_sketch_range((int64_t)ns, dJ, seed, dA, dO, dY, maxMW);
-    if (!rc) rc = jacobi_dispatch((int64_t)ns, yOff, M, Wd, v1, s1, dYo, dM, dW, dV1, dS1, dY, dV, dS);
-    /* the dispatcher left the small matrices' tables in place: the
-     * projection reads the sigma offsets of every matrix */
-    if (!rc) rc = bfk_h2d(dS1, s1, ns * 8);
-    if (!rc) rc = bfk_h2d(dW, Wd, ns * 4);
+    if (!rc) rc = jacobi_dispatch((int64_t)ns, yOff, M, Wd, dYo, dM, dW, dV1, dS1, dY, dV, dS);
     if (!rc) rc = bfk_sketch_project((int64_t)ns, dJ, dS1, dS, dA, dY, dB, dR, maxMW, maxNW, maxMN);
-    if (!rc) rc = jacobi_dispatch((int64_t)ns, bOff, N, Wd, v2, s2, dBo, dN, dW, dV2, dS2, dB, dV, dS);
+    if (!rc) rc = jacobi_dispatch((int64_t)ns, bOff, N, Wd, dBo, dN, dW, dV2, dS2, dB, dV, dS);
     if (!rc) rc = bfk_d2h(hY, dY, (size_t)tY * 16);
     if (!rc) rc = bfk_d2h(hB, dB, (size_t)tB * 16);
     if (!rc) rc = bfk_d2h(hV, dV, (size_t)tV * 16);
@@ -547,7 +612,7 @@ static int svd_batch_sketch(SvdJob *jobs, size_t nj, double tol, const int64_t *
   if (!rc && nf) { /* the full SVDs, rejected sketches included */
     SvdJob *fj = malloc(nf * sizeof(SvdJob));
     for (size_t x = 0; x < nf; ++x) fj[x] = jobs[full[x]];
-    rc = svd_batch(fj, nf, tol);
+    rc = svd_batch(fj, nf, tol, work);
     for (size_t x = 0; x < nf; ++x) {
       SvdJob *J = &jobs[full[x]];
       J->k = fj[x].k;
@@ -578,7 +643,7 @@ int bfhipSvdBatchedSketch(BfSize batch, BfSize const *m, BfSize const *n, BfComp
     wd[i] = (int64_t)width[i];
     off += jobs[i].m * jobs[i].n;
   }
-  int rc = svd_batch_sketch(jobs, batch, tol, wd, seed, fellBack);
+  int rc = svd_batch_sketch(jobs, batch, tol, wd, seed, fellBack, NULL);
   int64_t uo = 0, wo = 0;
   for (BfSize i = 0; i < batch; ++i) {
     if (!rc) {
@@ -610,13 +675,14 @@ typedef struct {
   BF_VEC(float) rank;
   int64_t numSvd, numSketched, numFell;
   uint64_t seed;
+  SvdWork work;
 } RankCtx;
 
 /* the SVDs of one round: with a model, widths from its predictions;
  * samples recorded afterwards */
 static int svd_round(RankCtx *rk, const BfFacSpec *spec, TreeView rt, int32_t colNode, const int32_t *rowNodes,
                      SvdJob *jobs, size_t nj) {
-  if (!rk || !rk->on || nj == 0) return svd_batch(jobs, nj, spec->tol);
+  if (!rk || !rk->on || nj == 0) return svd_batch(jobs, nj, spec->tol, rk ? &rk->work : NULL);
   float *f = malloc(nj * 6 * sizeof(float));
   const BfQuadtreeNode *cn = &rk->ct.nodes[colNode];
   const BfReal cb[4] = {cn->bboxMin[0], cn->bboxMin[1], cn->bboxMax[0], cn->bboxMax[1]};
@@ -639,9 +705,9 @@ static int svd_round(RankCtx *rk, const BfFacSpec *spec, TreeView rt, int32_t co
       const double p = pr[i] > 0 ? ceil((double)pr[i]) : 0;
       const int64_t mn = jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n;
       wd[i] = (int64_t)p + rk->oversample;
-      if (2 * wd[i] > mn || jobs[i].m * jobs[i].n < SVD_BIG_ENTRIES) wd[i] = 0;
+      if (2 * wd[i] > mn || jobs[i].m * jobs[i].n < SVD_QR_ENTRIES) wd[i] = 0;
     }
-    if (!rc) rc = svd_batch_sketch(jobs, nj, spec->tol, wd, rk->seed++, fell);
+    if (!rc) rc = svd_batch_sketch(jobs, nj, spec->tol, wd, rk->seed++, fell, &rk->work);
     for (size_t i = 0; i < nj && !rc; ++i) {
       const int64_t mn = jobs[i].m < jobs[i].n ? jobs[i].m : jobs[i].n;
       if (wd[i] > 0 && wd[i] < mn && wd[i] <= SVD_MAX_COLS) rk->numSketched += 1;
@@ -651,7 +717,7 @@ static int svd_round(RankCtx *rk, const BfFacSpec *spec, TreeView rt, int32_t co
     free(wd);
     free(fell);
   } else {
-    rc = svd_batch(jobs, nj, spec->tol);
+    rc = svd_batch(jobs, nj, spec->tol, &rk->work);
   }
   for (size_t i = 0; i < nj && !rc; ++i) {
     for (int q = 0; q < 6; ++q) BF_VEC_PUSH(rk->feat, f[6 * i + q]);
@@ -881,6 +947,7 @@ void bfFacStreamerInit(BfFacStreamer *s, BfFacSpec const *spec) {
   s->ct = tree_view(spec->colTree);
   s->rowRevPerm = spec->rowTree->perm ? bfPermGetReversePerm(spec->rowTree->perm) : NULL;
   size_t nc = count_nodes(s->ct, 0);
+  s->rank.work.locked = 1;
   s->post = malloc(nc * sizeof(int32_t));
   s->numPost = 0;
   post_order(s->ct, 0, s->post, &s->numPost);
@@ -900,6 +967,7 @@ void bfFacStreamerDeinit(BfFacStreamer *s) {
   free(s->facs);
   free(s->post);
   free(s->initCut);
+  svd_work_free(&s->rank.work);
   BF_VEC_FREE(s->rank.feat);
   BF_VEC_FREE(s->rank.rank);
   memset(s, 0, sizeof(*s));
