@@ -52,7 +52,7 @@ int bfk_set_compensation(int on);
 int bfk_sample(const BfkKernelJob *dJobs, int64_t numJobs, const double *dSrcXY, const double *dTgtXY,
                const double *dSrcN, const double *dTgtN, BfkLayer layer, double *dArena);
 int bfk_lstsq_begin(size_t maxOversizeBytes, int64_t numOversize);
-int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const int32_t *dOrder, int64_t numJobs, size_t ldsBytes,
+int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const uint32_t *dGroups, int64_t numGroups, size_t ldsBytes,
                      const double *dSrcXY, const double *dSrcN, BfkLayer layer, double *dArena);
 int bfk_lstsq_end(void);
 void bfk_set_lstsq_waves(int64_t two, int64_t four, int64_t *old2, int64_t *old4);

@@ -818,20 +818,31 @@ __device__ __forceinline__ LstsqView lstsq_view(double2 *base, int p, int n) {
   return L;
 }
 
-/* One job per block of T threads.  The working set lives in LDS, or for
- * jobs too large for LDS (about one in 10^4 at N = 2^20) in a per-block
- * slice of a global scratch buffer. */
+/* One group of jobs per block of T threads: 1 to 4 re-expansion blocks that
+ * invert the same matrix, written one after another (groups[]: first job <<
+ * 2 | jobs - 1), solved once against the columns of all: the time goes to
+ * latency-bound sweeps over the matrix (QR, then ~5 Jacobi sweeps), which the
+ * right parts of further blocks ride along (curve, N = 2^18, 1.9 blocks per
+ * group: 255 -> 194 ms; box, 2^14, 4 per group: 5.9 -> 3.45 ms).  The working set
+ * lives in LDS, or for jobs too large for LDS (about one in 10^4 at N = 2^20,
+ * never grouped) in a per-block slice of a global scratch buffer. */
 /* five waves per SIMD: the solve fits in 96 VGPRs without spills, and the
- * LDS of the common 8-12 KiB jobs allows about that many per CU anyway */
+ * LDS of the common 8-16 KiB groups allows about that many per CU anyway */
 template <int T, bool GLOBAL>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(5))) void k_lstsq(const BfkLstsqJob *__restrict__ jobs, const int32_t *__restrict__ order,
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(5))) void k_lstsq(const BfkLstsqJob *__restrict__ jobs,
+                                             const uint32_t *__restrict__ groups,
                                              const double2 *__restrict__ srcXY,
                                              const double2 *__restrict__ srcN, BfkLayer Lay,
                                              double2 *__restrict__ arena, double2 *__restrict__ gwork,
                                              int64_t gstride) {
   extern __shared__ double2 lds[];
-  const BfkLstsqJob J = jobs[order ? order[blockIdx.x] : blockIdx.x];
-  const int p = J.p, n = J.n, ld = p + n + 1;
+  const uint32_t grp = groups[blockIdx.x];
+  const BfkLstsqJob *jb = jobs + (grp >> 2);
+  const int nsub = (int)(grp & 3) + 1;
+  const BfkLstsqJob J = jb[0];
+  int n = J.n;
+  for (int q = 1; q < nsub; ++q) n += jb[q].n;
+  const int p = J.p, ld = p + n + 1;
   LstsqView L = lstsq_view(GLOBAL ? gwork + (int64_t)blockIdx.x * gstride : lds, p, n);
   double2 *tp = L.pts, *ep = tp + p, *op = ep + p;
   const int lane = threadIdx.x;
@@ -839,8 +850,14 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(5))) void k_l
     tp[i] = circle_pt(J.tcx, J.tcy, J.tr, p, i);
     ep[i] = circle_pt(J.ecx, J.ecy, J.er, p, i);
   }
-  for (int c = lane; c < n; c += T)
-    op[c] = J.origOff >= 0 ? srcXY[J.origOff + c] : circle_pt(J.ocx, J.ocy, J.orr, n, c);
+  for (int q = 0, c0 = 0; q < nsub; ++q) {
+    const BfkLstsqJob *O = jb + q;
+    const int on = O->n;
+    const int64_t off = O->origOff;
+    for (int c = lane; c < on; c += T)
+      op[c0 + c] = off >= 0 ? srcXY[off + c] : circle_pt(O->ocx, O->ocy, O->orr, on, c);
+    c0 += on;
+  }
   __syncthreads();
   const int W = p + n;
   /* entry e = i W + c; (i, c) advance by T entries without dividing */
@@ -850,9 +867,19 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(5))) void k_l
     if (c >= W) { c -= W; ++i; }
     double2 s = c < p ? ep[c] : op[c - p];
     double2 ns = make_double2(0, 0);
-    if (Lay.layer != 0)
-      ns = c < p ? circle_normal(J.ecx, J.ecy, J.er, s)
-                 : (J.origOff >= 0 ? srcN[J.origOff + c - p] : circle_normal(J.ocx, J.ocy, J.orr, s));
+    if (Lay.layer != 0) {
+      if (c < p) {
+        ns = circle_normal(J.ecx, J.ecy, J.er, s);
+      } else { /* of the job that holds column c */
+        const BfkLstsqJob *O = jb;
+        int oc = c - p;
+        for (int q = 1; q < nsub && oc >= O->n; ++q) {
+          oc -= O->n;
+          ++O;
+        }
+        ns = O->origOff >= 0 ? srcN[O->origOff + oc] : circle_normal(O->ocx, O->ocy, O->orr, s);
+      }
+    }
     L.M[i * ld + c] = green_call(Lay, J.k, tp[i], s, ns);
   }
   __syncthreads();
@@ -2677,24 +2704,22 @@ int bfk_lstsq_begin(size_t maxOversizeBytes, int64_t numOversize) {
   return 0;
 }
 
-/* One launch over `numJobs` jobs of one LDS class (ldsBytes per job):
- * dOrder[0..numJobs) indexes dJobs, or with dOrder NULL the jobs are
- * consecutive.  Launches rotate over g_stream and the side streams: a class of a
+/* One launch over `numGroups` groups of jobs of one LDS class (ldsBytes per
+ * group).  Launches rotate over g_stream and the side streams: a class of a
  * few large blocks runs for milliseconds at one block's latency and low
- * occupancy, and overlaps the classes that hold most of the blocks.  A job
+ * occupancy, and overlaps the classes that hold most of the blocks.  A group
  * gets 1, 2 or 4 waves by its class (g_lstsq2, g_lstsq4).  Jobs above the
  * LDS capacity run 256 threads each on the scratch of bfk_lstsq_begin,
  * chunk after chunk on g_stream. */
-int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const int32_t *dOrder, int64_t numJobs, size_t ldsBytes,
+int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const uint32_t *dGroups, int64_t numGroups, size_t ldsBytes,
                      const double *dSrcXY, const double *dSrcN, BfkLayer layer, double *dArena) {
-  if (numJobs <= 0) return 0;
+  if (numGroups <= 0) return 0;
   if (ldsBytes > g_ldsCap) {
     if (!g_lstsqWork || ldsBytes > g_lstsqWorkStride) return -3; /* bfk_lstsq_begin sized the scratch */
     const int64_t stride = (int64_t)(g_lstsqWorkStride / sizeof(double2));
-    for (int64_t j0 = 0; j0 < numJobs; j0 += BFK_SCRATCH_CHUNK) {
-      int64_t nj = numJobs - j0 < BFK_SCRATCH_CHUNK ? numJobs - j0 : BFK_SCRATCH_CHUNK;
-      hipLaunchKernelGGL((k_lstsq<256, true>), dim3((unsigned)nj), dim3(256), 0, g_stream,
-                         dOrder ? dJobs : dJobs + j0, dOrder ? dOrder + j0 : (const int32_t *)nullptr,
+    for (int64_t j0 = 0; j0 < numGroups; j0 += BFK_SCRATCH_CHUNK) {
+      int64_t nj = numGroups - j0 < BFK_SCRATCH_CHUNK ? numGroups - j0 : BFK_SCRATCH_CHUNK;
+      hipLaunchKernelGGL((k_lstsq<256, true>), dim3((unsigned)nj), dim3(256), 0, g_stream, dJobs, dGroups + j0,
                          (const double2 *)dSrcXY, (const double2 *)dSrcN, layer, (double2 *)dArena, g_lstsqWork,
                          stride);
       BFK_CHECK(hipGetLastError());
@@ -2704,20 +2729,19 @@ int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const int32_t *dOrder, int64_t nu
   hipStream_t st = g_nextStream == 0 ? g_stream : g_side[g_nextStream - 1];
   g_nextStream = (g_nextStream + 1) % (BFK_SIDE_STREAMS + 1);
   const int64_t maxGrid = 1 << 30;
-  for (int64_t j0 = 0; j0 < numJobs; j0 += maxGrid) {
-    int64_t nj = numJobs - j0 < maxGrid ? numJobs - j0 : maxGrid;
-    const BfkLstsqJob *jb = dOrder ? dJobs : dJobs + j0;
-    const int32_t *ob = dOrder ? dOrder + j0 : (const int32_t *)nullptr;
+  for (int64_t j0 = 0; j0 < numGroups; j0 += maxGrid) {
+    int64_t nj = numGroups - j0 < maxGrid ? numGroups - j0 : maxGrid;
+    const uint32_t *gb = dGroups + j0;
     if (ldsBytes > g_lstsq4)
-      hipLaunchKernelGGL((k_lstsq<256, false>), dim3((unsigned)nj), dim3(256), ldsBytes, st, jb, ob,
+      hipLaunchKernelGGL((k_lstsq<256, false>), dim3((unsigned)nj), dim3(256), ldsBytes, st, dJobs, gb,
                          (const double2 *)dSrcXY, (const double2 *)dSrcN, layer, (double2 *)dArena,
                          (double2 *)nullptr, (int64_t)0);
     else if (ldsBytes > g_lstsq2)
-      hipLaunchKernelGGL((k_lstsq<128, false>), dim3((unsigned)nj), dim3(128), ldsBytes, st, jb, ob,
+      hipLaunchKernelGGL((k_lstsq<128, false>), dim3((unsigned)nj), dim3(128), ldsBytes, st, dJobs, gb,
                          (const double2 *)dSrcXY, (const double2 *)dSrcN, layer, (double2 *)dArena,
                          (double2 *)nullptr, (int64_t)0);
     else
-      hipLaunchKernelGGL((k_lstsq<64, false>), dim3((unsigned)nj), dim3(64), ldsBytes, st, jb, ob,
+      hipLaunchKernelGGL((k_lstsq<64, false>), dim3((unsigned)nj), dim3(64), ldsBytes, st, dJobs, gb,
                          (const double2 *)dSrcXY, (const double2 *)dSrcN, layer, (double2 *)dArena,
                          (double2 *)nullptr, (int64_t)0);
     BFK_CHECK(hipGetLastError());
@@ -2725,8 +2749,9 @@ int bfk_lstsq_launch(const BfkLstsqJob *dJobs, const int32_t *dOrder, int64_t nu
   return 0;
 }
 
-/* the LDS classes (bytes per job) above which the compression runs 2 and
- * 4 waves per job; a negative value leaves that threshold as it is.  The
+/* the LDS classes (bytes per group) above which the compression runs 2 and
+ * 4 waves per group (16 and 40 KiB: 12 or 20 KiB for two waves are within 1%
+ * at N = 2^18 and 2^20, 64 KiB for four costs 4%); a negative value leaves that threshold as it is.  The
  * previous values go to *old2 / *old4 when given. */
 void bfk_set_lstsq_waves(int64_t two, int64_t four, int64_t *old2, int64_t *old4) {
   if (old2) *old2 = (int64_t)g_lstsq2;

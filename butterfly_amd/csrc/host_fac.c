@@ -481,21 +481,37 @@ static void *apply_plan_task(void *arg) {
   return NULL;
 }
 
-/* Parallel stable counting sort of the re-expansion jobs by LDS class,
- * largest class first, writing the jobs themselves (no order array): each
- * of NT threads classes a contiguous range and counts it, the class starts
- * are summed per thread, then each thread scatters its range.  Within a
- * class the jobs keep plan order, as group_by_class(..., 1) with a gather
- * would give. */
-enum { CLASS_NT = 16 };
+/* The re-expansion blocks of one row of a factor invert the same matrix
+ * (same test and equivalent circles) and lie one after another in the arena:
+ * up to LSTSQ_GROUP of them, as many as fit in LDS together, become one group,
+ * sampled, factored and rotated once against all their columns (a block has
+ * at most four children, so a longer run does not occur in a row).  Blocks
+ * solved one by one / grouped: 5.9 / 3.45 ms (box, N = 2^14), 255 / 194 ms
+ * (curve, 2^18), 1036 / 861 ms (curve, 2^20).  All of LDS is let to a group:
+ * with at most 80 / 52 / 40 / 24 KiB the curve at 2^18 takes 199 / 202 / 206 /
+ * 212 ms, the box the same within 2%. */
+enum { CLASS_NT = 16, LSTSQ_GROUP = 4 };
 
+static int same_matrix(const BfkLstsqJob *a, const BfkLstsqJob *b) {
+  return a->p == b->p && a->ecx == b->ecx && a->ecy == b->ecy && a->er == b->er && a->tcx == b->tcx &&
+         a->tcy == b->tcy && a->tr == b->tr && a->k == b->k && a->rcond == b->rcond &&
+         b->out == a->out + (int64_t)a->p * a->n;
+}
+
+/* Parallel stable counting sort of the groups by LDS class, largest class
+ * first, writing the jobs themselves, a group's one after another, and the
+ * groups (first job << 2 | jobs - 1): each of NT threads groups and classes a
+ * contiguous range and counts it, the class starts are summed per thread,
+ * then each thread scatters its range.  Within a class the groups keep plan
+ * order. */
 typedef struct {
   const BfkLstsqJob *src;
   BfkLstsqJob *dst;
-  uint32_t *cls;
-  size_t i0, i1;
+  uint32_t *grp; /* the groups, in class order */
+  uint32_t *cls; /* class << 3 | jobs at a group's first job */
+  size_t i0, i1, cap;
   uint32_t maxCls;
-  size_t *pos; /* per class: the next slot of this thread (phase 3), counts (phase 2) */
+  size_t *pos, *gpos; /* per class: the next job / group slot of this thread (phase 3), counts (phase 2) */
   int phase;
 } ClassTask;
 
@@ -503,16 +519,33 @@ static void *class_task(void *arg) {
   ClassTask *t = arg;
   if (t->phase == 1) {
     uint32_t mx = 0;
-    for (size_t i = t->i0; i < t->i1; ++i) {
-      const uint32_t c = (uint32_t)((BF_LSTSQ_UNITS(t->src[i].p, t->src[i].n) * 16 + 4095) >> 12);
-      t->cls[i] = c;
+    for (size_t i = t->i0; i < t->i1;) {
+      const BfkLstsqJob *J = &t->src[i];
+      int64_t n = J->n;
+      size_t j = i + 1;
+      while (j < t->i1 && j < i + LSTSQ_GROUP && same_matrix(&t->src[j - 1], &t->src[j]) &&
+             BF_LSTSQ_UNITS(J->p, n + t->src[j].n) * 16 <= t->cap)
+        n += t->src[j++].n;
+      const uint32_t c = (uint32_t)((BF_LSTSQ_UNITS(J->p, n) * 16 + 4095) >> 12);
+      t->cls[i] = c << 3 | (uint32_t)(j - i);
       if (c > mx) mx = c;
+      i = j;
     }
     t->maxCls = mx;
   } else if (t->phase == 2) {
-    for (size_t i = t->i0; i < t->i1; ++i) ++t->pos[t->cls[i]];
+    for (size_t i = t->i0; i < t->i1; i += t->cls[i] & 7) {
+      t->pos[t->cls[i] >> 3] += t->cls[i] & 7;
+      ++t->gpos[t->cls[i] >> 3];
+    }
   } else {
-    for (size_t i = t->i0; i < t->i1; ++i) t->dst[t->pos[t->cls[i]]++] = t->src[i];
+    for (size_t i = t->i0; i < t->i1;) {
+      const uint32_t c = t->cls[i] >> 3, n = t->cls[i] & 7;
+      const size_t d = t->pos[c];
+      t->grp[t->gpos[c]++] = (uint32_t)(d << 2) | (n - 1);
+      for (uint32_t q = 0; q < n; ++q) t->dst[d + q] = t->src[i + q];
+      t->pos[c] = d + n;
+      i += n;
+    }
   }
   return NULL;
 }
@@ -530,9 +563,11 @@ static void class_phase(ClassTask *t, int nt, int phase) {
     if (ok[q]) pthread_join(th[q], NULL);
 }
 
-/* dst gets src's jobs class by class (largest first); gs gets each
- * non-empty class's first position plus a final nj, gb its byte size */
-static int class_sort_jobs(const BfkLstsqJob *src, size_t nj, BfkLstsqJob *dst, BfI64Vec *gs, BfSizeVec *gb) {
+/* dst gets src's jobs class by class (largest first) and grp the groups;
+ * gs gets each non-empty class's first group plus a final count, gb its byte
+ * size */
+static int class_sort_jobs(const BfkLstsqJob *src, size_t nj, BfkLstsqJob *dst, uint32_t *grp, BfI64Vec *gs,
+                           BfSizeVec *gb) {
   ClassTask t[CLASS_NT];
   const int nt = nj < ((size_t)1 << 16) ? 1 : CLASS_NT;
   uint32_t *cls = malloc((nj ? nj : 1) * sizeof(uint32_t));
@@ -542,37 +577,50 @@ static int class_sort_jobs(const BfkLstsqJob *src, size_t nj, BfkLstsqJob *dst, 
   for (int q = 0; q < nt; ++q) {
     t[q].src = src;
     t[q].dst = dst;
+    t[q].grp = grp;
     t[q].cls = cls;
-    t[q].i0 = nj * (size_t)q / (size_t)nt;
-    t[q].i1 = nj * (size_t)(q + 1) / (size_t)nt;
+    t[q].cap = bfk_lds_cap();
+    /* a range starts where the matrix changes, so that the groups do not
+     * depend on the ranges */
+    size_t i = nj * (size_t)q / (size_t)nt;
+    while (i > 0 && i < nj && same_matrix(&src[i - 1], &src[i])) ++i;
+    t[q].i0 = i;
+    if (q) t[q - 1].i1 = i;
   }
+  t[nt - 1].i1 = nj;
   class_phase(t, nt, 1);
   uint32_t maxCls = 0;
   for (int q = 0; q < nt; ++q)
     if (t[q].maxCls > maxCls) maxCls = t[q].maxCls;
-  size_t *pos = calloc((size_t)nt * (maxCls + 1), sizeof(size_t));
+  const size_t nc = (size_t)maxCls + 1;
+  size_t *pos = calloc(2 * (size_t)nt * nc, sizeof(size_t));
   if (!pos) {
     free(cls);
     return -2;
   }
-  for (int q = 0; q < nt; ++q) t[q].pos = pos + (size_t)q * (maxCls + 1);
+  for (int q = 0; q < nt; ++q) {
+    t[q].pos = pos + (size_t)q * nc;
+    t[q].gpos = pos + (size_t)(nt + q) * nc;
+  }
   class_phase(t, nt, 2);
-  /* counts -> each thread's first slot per class, classes descending */
+  /* counts -> each thread's first slots per class, classes descending */
   gs->n = gb->n = 0;
-  size_t run = 0;
+  size_t run = 0, grun = 0;
   for (int64_t c = maxCls; c >= 0; --c) {
-    const size_t first = run;
+    const size_t first = grun;
     for (int q = 0; q < nt; ++q) {
-      const size_t cnt = t[q].pos[c];
+      const size_t cnt = t[q].pos[c], gcnt = t[q].gpos[c];
       t[q].pos[c] = run;
+      t[q].gpos[c] = grun;
       run += cnt;
+      grun += gcnt;
     }
-    if (run > first) {
+    if (grun > first) {
       BF_VEC_PUSH(*gs, (int64_t)first);
       BF_VEC_PUSH(*gb, (size_t)c << 12);
     }
   }
-  BF_VEC_PUSH(*gs, (int64_t)nj);
+  BF_VEC_PUSH(*gs, (int64_t)grun);
   class_phase(t, nt, 3);
   free(pos);
   free(cls);
@@ -605,14 +653,18 @@ static int run_factor_kernels(BfMatHipButterfly *F, double *tApplyPlan) {
   BfSizeVec gb;
   memset(&gs, 0, sizeof(gs));
   memset(&gb, 0, sizeof(gb));
+  if (nj >> 30) return -2; /* a group holds its first job's index in 30 bits */
   BfkLstsqJob *sorted = malloc((nj ? nj : 1) * sizeof(BfkLstsqJob));
+  uint32_t *grp = malloc((nj ? nj : 1) * sizeof(uint32_t));
   bfHugePages(sorted, nj * sizeof(BfkLstsqJob));
-  if (!sorted || class_sort_jobs(F->lstsqJobs.a, nj, sorted, &gs, &gb)) {
+  if (!sorted || !grp || class_sort_jobs(F->lstsqJobs.a, nj, sorted, grp, &gs, &gb)) {
     free(sorted);
+    free(grp);
     BF_VEC_FREE(gs);
     BF_VEC_FREE(gb);
     return -2;
   }
+  const size_t ng = (size_t)gs.a[gs.n - 1];
   bfTrace("factor: jobs sorted by class", tk);
   /* the apply plan is host work: build it on a helper thread while this
    * thread uploads the jobs and the kernels run */
@@ -623,7 +675,8 @@ static int run_factor_kernels(BfMatHipButterfly *F, double *tApplyPlan) {
   /* uploaded in chunks on the copy stream; each uploaded range is launched
    * at once, so the upload (several GB for large or batched problems)
    * overlaps the kernels */
-  BfkLstsqJob *dL = bfk_malloc((nj ? nj : 1) * sizeof(BfkLstsqJob));
+  BfkLstsqJob *dL = bfk_malloc((nj ? nj : 1) * sizeof(BfkLstsqJob) + (ng ? ng : 1) * sizeof(uint32_t));
+  uint32_t *dG = (uint32_t *)(dL + nj);
   if (!dL) rc = -2;
   /* jobs above the LDS capacity share one scratch buffer */
   size_t bigBytes = 0;
@@ -638,15 +691,25 @@ static int run_factor_kernels(BfMatHipButterfly *F, double *tApplyPlan) {
   /* jobs per upload: small at first so that the kernels start early, then
    * doubling up to 4M */
   size_t chunk = (size_t)1 << 18;
-  size_t up = 0, launched = 0, g = 0;
+  size_t up = 0, launched = 0, g = 0; /* jobs uploaded, groups launched, class */
   while (!rc && up < nj) {
     const size_t n = nj - up < chunk ? nj - up : chunk;
     if (chunk < ((size_t)1 << 22)) chunk *= 2;
     rc = bfk_h2d_side(dL + up, sorted + up, n * sizeof(BfkLstsqJob));
     up += n;
+    /* the groups whose jobs are up: their last job lies before `up` */
+    size_t lo = launched, hi = ng;
+    while (lo < hi) {
+      const size_t mid = (lo + hi) / 2;
+      if ((grp[mid] >> 2) + (grp[mid] & 3) < up) lo = mid + 1;
+      else hi = mid;
+    }
+    const size_t ready = lo;
+    if (!rc && ready > launched)
+      rc = bfk_h2d_side(dG + launched, grp + launched, (ready - launched) * sizeof(uint32_t));
     /* what is uploaded: the rest of the current class, the classes that
      * are complete, and the uploaded start of the next */
-    while (!rc && g + 1 < gs.n && launched < up) {
+    while (!rc && g + 1 < gs.n && launched < ready) {
       /* classes [g, gEnd): one class, or all the classes above the LDS
        * capacity (they come first and share the scratch, whose stride fits
        * the largest, so they go out in one launch: per class they were ~40
@@ -657,8 +720,8 @@ static int run_factor_kernels(BfMatHipButterfly *F, double *tApplyPlan) {
         lds = bigBytes;
       }
       const size_t classEnd = (size_t)gs.a[gEnd];
-      const size_t end = classEnd < up ? classEnd : up;
-      rc = bfk_lstsq_launch(dL + launched, NULL, (int64_t)(end - launched), lds, F->dSrcXY, F->dSrcN, proxyLayer,
+      const size_t end = classEnd < ready ? classEnd : ready;
+      rc = bfk_lstsq_launch(dL, dG + launched, (int64_t)(end - launched), lds, F->dSrcXY, F->dSrcN, proxyLayer,
                             F->dArena);
       launched = end;
       if (launched == classEnd) g = gEnd;
@@ -672,6 +735,7 @@ static int run_factor_kernels(BfMatHipButterfly *F, double *tApplyPlan) {
     if (!rc) rc = rc2;
   }
   free(sorted);
+  free(grp);
   if (threaded) pthread_join(th, NULL);
   bfTrace("factor: apply plan joined", tk);
   *tApplyPlan = task.seconds;
