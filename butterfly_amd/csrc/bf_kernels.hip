@@ -2048,6 +2048,31 @@ static int g_applyWaves = 1;
 static int g_mfmaCT = -1;
 #define MFMA_DEFAULT_F64 (2 | 16)
 #define MFMA_DEFAULT_F32 2
+/* waves at most per segment of a split stage, and the LDS bytes of one wave's
+ * 16 x 16 tile of complex sums */
+#define MFMA_SPLIT_MAX 8
+#define MFMA_SPLIT_TILE 4096
+/* A stage of few segments leaves the chip idle while each wave walks a long
+ * chain.  Its row passes go to waves of their own while the segments (times
+ * column chunks) number under 16384, two per wave slot in use; then, while
+ * there are fewer than 2048 such waves, 2 to 8 of them share the columns of
+ * one pass (at least 8 steps of 4 each).  16 right-hand sides, one wave per
+ * segment / row passes split / columns split too: 16 problems of 4096-65536
+ * points in FP32 1187 / 1087 / 1087 us, box of 16384 points FP64 219 / 201 /
+ * 198 us, FP32 183 / 145 / 145 us; curve of 4096 points FP32 236 / 127 / 108
+ * us, of 5000 points with 20 in FP64 374 / 266 / 242 us.  Row passes split at
+ * 32768 and 65536 segments cost the curve of 100003 points 2.5 and 14% (a
+ * segment's passes share its inputs in L1), the columns split at 4096 waves
+ * the box 8%. */
+static int mfma_row_groups(int64_t numSegs, const BfkStageShape &sh, int chunks, int rowTiles) {
+  return numSegs * chunks < 16384 ? (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles) : 1;
+}
+static int mfma_split(int64_t numSegs, const BfkStageShape &sh, int items, int tiles) {
+  const int64_t steps = numSegs > 0 ? sh.cols / numSegs / 4 : 0;
+  int w = 1;
+  while (tiles <= 4 && w < MFMA_SPLIT_MAX && w * tiles < 16 && numSegs * items * w < 2048 && steps >= 16 * w) w *= 2;
+  return w;
+}
 /* the default shape with no more column tiles than nrhs fills */
 static inline int mfma_auto(int cfg, int nrhs) {
   int ct = cfg & 15;
@@ -2066,10 +2091,11 @@ __constant__ int g_foldMaskDev = 0;
 
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
 #define MFMA_SEG_GROUP 4
-/* workgroups of one many-RHS stage: every (segment, column chunk) pair */
-static inline unsigned mfma_grid(int64_t numSegs, int chunks) {
+/* workgroups of one many-RHS stage: every segment's items (column chunks
+ * times row groups) */
+static inline unsigned mfma_grid(int64_t numSegs, int items) {
   const int64_t g = 8 * MFMA_SEG_GROUP;
-  return (unsigned)(((numSegs + g - 1) / g) * g * chunks);
+  return (unsigned)(((numSegs + g - 1) / g) * g * items);
 }
 
 /* 16x16x4 MFMA on one wave, real operands.  Operand lanes: A[l%16][l/16],
@@ -2111,7 +2137,15 @@ struct MfmaF32 {
 
 /* One stage of the apply for nrhs right-hand sides on the matrix cores:
  * one wave computes RT x 16 rows x 16*CT columns of a segment's output per
- * pass.  The complex product is four real MFMAs per 16x16x4 step (re*re -
+ * pass, every rowGroups-th pass of the segment; with SPLIT the workgroup's
+ * waves share a pass's columns and the first adds their sums up.  Most
+ * segments are one pass of about ten steps, so a wave's life is the chain
+ * segment -> term -> operands -> result and the start is kept short: the
+ * terms are walked once, the first block term's record is kept and the next
+ * one's loaded while the current term's columns are (16 right-hand sides on
+ * 100003 points in FP32 1495 -> 1400 us, 64 on 30000 1270 -> 1160 us, 16
+ * problems of 4096-65536 points 1087 -> 1005 us against walking them three
+ * times).  The complex product is four real MFMAs per 16x16x4 step (re*re -
  * im*im, re*im + im*re); with RT = 2 every input value a lane loads feeds
  * both row tiles (segments are mostly 17-22 rows high), which halves the
  * reads of the input vectors.  blockIdx.x picks the column chunk so the
@@ -2130,13 +2164,13 @@ struct MfmaF32 {
  * added into FP64 sums every (mask + 1) steps and at the end of every
  * term, so rounding no longer grows with the length of the rows. */
 #define MFMA_RING 3
-template <class M, int CT, int RT, bool LO, bool COMP>
-__global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ segs,
+template <class M, int CT, int RT, bool LO, bool COMP, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * MFMA_SPLIT_MAX : 64) void k_applyN_mfma(const BfkSeg *__restrict__ segs,
                                                     const BfkTerm *__restrict__ terms,
                                                     const typename M::V *__restrict__ hi,
                                                     const typename M::V *__restrict__ lo,
                                                     typename BufsOf<typename M::V>::T bufs, int nrhs,
-                                                    int numChunks, int64_t numSegs) {
+                                                    int numChunks, int rowGroups, int64_t numSegs) {
   typedef typename M::V V;
   typedef typename M::Acc Acc;
   /* workgroups go to the 8 XCDs round-robin by id: ids b with the same
@@ -2145,26 +2179,46 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
    * chunks gets the ids 8 * slot + xcd, so both the blocks and the inputs
    * they share are read from one L2. */
   const int64_t slot = blockIdx.x >> 3;
-  const int64_t per = (int64_t)MFMA_SEG_GROUP * numChunks;
+  const int items = numChunks * rowGroups;
+  const int64_t per = (int64_t)MFMA_SEG_GROUP * items;
   const int64_t grp = slot / per;
   const int64_t within = slot - grp * per;
-  const int64_t si = (grp * 8 + (blockIdx.x & 7)) * MFMA_SEG_GROUP + within / numChunks;
-  const int chunk = (int)(within - (within / numChunks) * numChunks);
+  const int64_t si = (grp * 8 + (blockIdx.x & 7)) * MFMA_SEG_GROUP + within / items;
+  const int item = (int)(within - (within / items) * items);
+  const int rowGroup = item / numChunks, chunk = item - rowGroup * numChunks;
   if (si >= numSegs) return;
   const BfkSeg Sg = segs[si];
-  const int l = threadIdx.x;
+  const int l = threadIdx.x & 63;
+  const int wv = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int c0 = chunk * 16 * CT;
   const int m = Sg.m;
+  if (rowGroup * 16 * RT >= m) return;
   const int lr = l & 15, lk = l >> 4;
   V *y = bufs.out[Sg.ybuf];
   int steps = 0; /* 4-column steps over the block terms */
+  int first = Sg.t1, idents = 0; /* the first block term with columns, the identity terms */
+  BfkTerm FT = {};
   for (int t = Sg.t0; t < Sg.t1; ++t) {
     const BfkTerm T = terms[t];
-    if (T.aOff >= 0) steps += (T.n + 3) >> 2;
+    if (T.aOff < 0) {
+      ++idents;
+      continue;
+    }
+    if (steps == 0) {
+      first = t;
+      FT = T;
+    }
+    steps += (T.n + 3) >> 2;
+  }
+  int skip = 0; /* the steps before this wave's */
+  if constexpr (SPLIT) {
+    const int nw = (int)blockDim.x >> 6;
+    skip = (int)((int64_t)steps * wv / nw);
+    steps = (int)((int64_t)steps * (wv + 1) / nw) - skip;
   }
   int colc[CT];
   for (int q = 0; q < CT; ++q) colc[q] = min(c0 + 16 * q + lr, nrhs - 1);
-  for (int rt = 0; rt < m; rt += 16 * RT) {
+  for (int rt = rowGroup * 16 * RT; rt < m; rt += 16 * RT * rowGroups) {
     /* row tiles of this pass that hold rows (uniform) */
     const int live = min(RT, (m - rt + 15) >> 4);
     Acc re[RT][CT], im[RT][CT], pre[RT][CT], pim[RT][CT];
@@ -2175,7 +2229,7 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
           re[u][q][r] = im[u][q][r] = pre[u][q][r] = pim[u][q][r] = 0;
           re64[u][q][r] = im64[u][q][r] = 0;
         }
-    for (int t = Sg.t0; t < Sg.t1; ++t) { /* identity terms */
+    for (int t = idents != 0 && wv == 0 ? Sg.t0 : Sg.t1; t < Sg.t1; ++t) { /* identity terms */
       const BfkTerm T = terms[t];
       if (T.aOff >= 0) continue;
       const V *x = bufs.in[T.xbuf];
@@ -2207,11 +2261,17 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
       int arow[RT];
       for (int u = 0; u < RT; ++u) arow[u] = min(rt + 16 * u + lr, m - 1);
       /* the load cursor: term lt, its columns from lk0 */
-      int lt = Sg.t0; /* the first block term with columns (steps > 0: one exists) */
-      while (terms[lt].aOff < 0 || terms[lt].n <= 0) ++lt;
-      BfkTerm LT = terms[lt];
+      int lt = first, lk0 = 4 * skip; /* the term and column of step `skip` */
+      BfkTerm LT = FT;
+      if constexpr (SPLIT)
+        while (LT.aOff < 0 || LT.n <= lk0) { /* steps > 0: it exists */
+          if (LT.aOff >= 0) lk0 -= (LT.n + 3) & ~3;
+          LT = terms[++lt];
+        }
+      /* the next term's record is on its way while this one's columns load */
+      BfkTerm NT = terms[min(lt + 1, Sg.t1 - 1)];
       const V *LX = bufs.in[LT.xbuf];
-      int lk0 = 0, issued = 0;
+      int issued = 0, done = 0;
       V ra[MFMA_RING][RT], rl[MFMA_RING][RT], rb[MFMA_RING][CT];
       int sk0[MFMA_RING], sn[MFMA_RING];
       auto issue = [&](int s) {
@@ -2229,9 +2289,11 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
           lk0 += 4;
           if (lk0 >= LT.n) {
             lk0 = 0;
-            do ++lt;
-            while (terms[lt].aOff < 0 || terms[lt].n <= 0);
-            LT = terms[lt];
+            do {
+              LT = NT;
+              ++lt;
+              NT = terms[min(lt + 1, Sg.t1 - 1)];
+            } while (LT.aOff < 0 || LT.n <= 0);
             LX = bufs.in[LT.xbuf];
           }
         }
@@ -2244,6 +2306,7 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
         }
         for (int q = 0; q < CT; ++q) b[q] = rb[s][q];
         const int rem = sn[s] - sk0[s];
+        const bool last = SPLIT && ++done == steps; /* a wave's last step folds like a term's */
         if (rem < 4 && lk >= rem) {
           for (int u = 0; u < RT; ++u) {
             a[u] = czero<V>();
@@ -2269,7 +2332,7 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
             di = M::mma(ai, b[q].x, di);
           }
           if constexpr (COMP) {
-            if (((sk0[s] >> 2) & g_foldMaskDev) == g_foldMaskDev || rem <= 4)
+            if (((sk0[s] >> 2) & g_foldMaskDev) == g_foldMaskDev || rem <= 4 || last)
               for (int q = 0; q < CT; ++q) {
                 re64[u][q] += __builtin_convertvector(pre[u][q], mf_d4);
                 im64[u][q] += __builtin_convertvector(pim[u][q], mf_d4);
@@ -2302,6 +2365,43 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
       for (int s = 0; s < MFMA_RING - 1; ++s)
         if (s < tail) compute(s);
     }
+    if constexpr (SPLIT) { /* the first wave adds the others' sums */
+      typedef typename std::conditional<COMP, double, typename M::S>::type R;
+      extern __shared__ double2 lds[];
+      const int nw = (int)blockDim.x >> 6;
+      R *red = (R *)lds + l;
+      auto cell = [&](int w, int u, int q, int r) { return ((((w - 1) * RT + u) * CT + q) * 4 + r) * 128; };
+      if (wv != 0)
+        for (int u = 0; u < RT; ++u)
+          for (int q = 0; q < CT; ++q)
+            for (int r = 0; r < 4; ++r) {
+              R *p = red + cell(wv, u, q, r);
+              if constexpr (COMP) {
+                p[0] = re64[u][q][r];
+                p[64] = im64[u][q][r];
+              } else {
+                p[0] = re[u][q][r];
+                p[64] = im[u][q][r];
+              }
+            }
+      __syncthreads();
+      if (wv == 0)
+        for (int w = 1; w < nw; ++w)
+          for (int u = 0; u < RT; ++u)
+            for (int q = 0; q < CT; ++q)
+              for (int r = 0; r < 4; ++r) {
+                const R *p = red + cell(w, u, q, r);
+                if constexpr (COMP) {
+                  re64[u][q][r] += p[0];
+                  im64[u][q][r] += p[64];
+                } else {
+                  re[u][q][r] += p[0];
+                  im[u][q][r] += p[64];
+                }
+              }
+      __syncthreads(); /* before the next pass writes its sums */
+      if (wv != 0) continue;
+    }
     for (int u = 0; u < RT; ++u)
       for (int q = 0; q < CT; ++q) {
         const int col = c0 + 16 * q + lr;
@@ -2327,23 +2427,37 @@ __global__ __launch_bounds__(64) void k_applyN_mfma(const BfkSeg *__restrict__ s
  * right-hand sides per wave (1, 2, 4 or 8) | 16 for two row tiles per
  * wave */
 template <class M, bool LO, bool COMP>
-static void launch_mfma(int cfg, dim3 grid, const BfkSeg *segs, const BfkTerm *terms, const typename M::V *H,
-                        const typename M::V *Lo, typename BufsOf<typename M::V>::T b, int nrhs, int chunks,
+static void launch_mfma(int cfg, const BfkSeg *segs, const BfkStageShape &shape, const BfkTerm *terms,
+                        const typename M::V *H, const typename M::V *Lo, typename BufsOf<typename M::V>::T b, int nrhs,
                         int64_t numSegs) {
-#define BFK_MFMA_LAUNCH(C, R)                                                                                  \
-  hipLaunchKernelGGL((k_applyN_mfma<M, C, R, LO, COMP>), grid, dim3(64), 0, g_stream, segs, terms, H, Lo, b, nrhs, \
-                     chunks, numSegs)
-  const int ct = cfg & 15;
-  if ((cfg & 16) && ct != 8) {
+  const int ct = cfg & 15, rts = (cfg & 16) && ct != 8 ? 2 : 1;
+  const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
+  const int groups = mfma_row_groups(numSegs, shape, chunks, rts);
+  const dim3 grid(mfma_grid(numSegs, chunks * groups));
+  const int w = mfma_split(numSegs, shape, chunks * groups, rts * ct);
+#define BFK_MFMA_LAUNCH1(C, R)                                                                                       \
+  hipLaunchKernelGGL((k_applyN_mfma<M, C, R, LO, COMP, false>), grid, dim3(64), 0, g_stream, segs, terms, H, Lo, b, \
+                     nrhs, chunks, groups, numSegs)
+#define BFK_MFMA_LAUNCH(C, R)                                                                                \
+  do {                                                                                                       \
+    if (w > 1)                                                                                               \
+      hipLaunchKernelGGL((k_applyN_mfma<M, C, R, LO, COMP, true>), grid, dim3(64 * w),                       \
+                         (size_t)(w - 1) * R * C * MFMA_SPLIT_TILE, g_stream, segs, terms, H, Lo, b, nrhs,    \
+                         chunks, groups, numSegs);                                                           \
+    else                                                                                                     \
+      BFK_MFMA_LAUNCH1(C, R);                                                                                \
+  } while (0)
+  if (rts == 2) {
     if (ct == 1) BFK_MFMA_LAUNCH(1, 2);
     else if (ct == 2) BFK_MFMA_LAUNCH(2, 2);
-    else BFK_MFMA_LAUNCH(4, 2);
+    else BFK_MFMA_LAUNCH1(4, 2);
   } else {
     if (ct == 1) BFK_MFMA_LAUNCH(1, 1);
     else if (ct == 2) BFK_MFMA_LAUNCH(2, 1);
-    else if (ct == 8) BFK_MFMA_LAUNCH(8, 1);
-    else BFK_MFMA_LAUNCH(4, 1);
+    else if (ct == 8) BFK_MFMA_LAUNCH1(8, 1);
+    else BFK_MFMA_LAUNCH1(4, 1);
   }
+#undef BFK_MFMA_LAUNCH1
 #undef BFK_MFMA_LAUNCH
 }
 
@@ -3070,10 +3184,7 @@ static int launch_stage_f64(const BfkSeg *segs, int64_t n, const BfkStageShape &
   if (n == 0) return 0;
   if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
     const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F64, nrhs);
-    const int ct = mc & 15;
-    const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
-    dim3 grid(mfma_grid(n, chunks));
-    launch_mfma<MfmaF64, false, false>(mc, grid, segs, dTerms, (const double2 *)dArena, nullptr, b, nrhs, chunks, n);
+    launch_mfma<MfmaF64, false, false>(mc, segs, shape, dTerms, (const double2 *)dArena, nullptr, b, nrhs, n);
     BFK_CHECK(hipGetLastError());
   } else {
     const int wv = nrhs == 1 && cfg >= 0 ? cfg & 15 : g_applyWaves;
@@ -3271,16 +3382,13 @@ static int launch_stage_f32(const BfkSeg *segs, int64_t n, const BfkStageShape &
   const float2 *H = (const float2 *)dArenaHi, *Lo = (const float2 *)dArenaLo;
   if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
     const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F32, nrhs);
-    const int ct = mc & 15;
-    const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
-    dim3 grid(mfma_grid(n, chunks));
     if (Lo) { /* hi + lo summed in FP64 on load, the FP64 matrix cores */
-      launch_mfma<MfmaF64S32, true, false>(mc, grid, segs, dTerms, H, Lo, b, nrhs, chunks, n);
+      launch_mfma<MfmaF64S32, true, false>(mc, segs, shape, dTerms, H, Lo, b, nrhs, n);
     } else if (g_comp32 == 1) {
-      launch_mfma<MfmaF64S32, false, false>(mc, grid, segs, dTerms, H, nullptr, b, nrhs, chunks, n);
+      launch_mfma<MfmaF64S32, false, false>(mc, segs, shape, dTerms, H, nullptr, b, nrhs, n);
     } else {
-      if (g_comp32) launch_mfma<MfmaF32, false, true>(mc, grid, segs, dTerms, H, Lo, b, nrhs, chunks, n);
-      else launch_mfma<MfmaF32, false, false>(mc, grid, segs, dTerms, H, Lo, b, nrhs, chunks, n);
+      if (g_comp32) launch_mfma<MfmaF32, false, true>(mc, segs, shape, dTerms, H, Lo, b, nrhs, n);
+      else launch_mfma<MfmaF32, false, false>(mc, segs, shape, dTerms, H, Lo, b, nrhs, n);
     }
     BFK_CHECK(hipGetLastError());
   } else {
