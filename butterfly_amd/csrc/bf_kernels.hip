@@ -3179,11 +3179,37 @@ int bfk_ortho(const BfkOrthoJob *dJobs, const int32_t *dOrder, int numGroups, co
  * it is not used. */
 static int g_capturing = 0; /* launches go into a graph: no timing events */
 
+/* Whether a stage runs on the matrix cores: from 16 right-hand sides on
+ * unless its launch shape or the global setting says otherwise, and below 16
+ * from `least` on, where the 16 padded columns cost less than the vector
+ * unit's.  us per apply at 5 / 6 / 8 / 12 right-hand sides, vector unit then
+ * matrix cores: curve of 100003 points FP64 1670 / 1922 / 2708 / 3768 and 1614 /
+ * 1637 / 1725 / 1926, FP32 1375 / 1480 / 2016 / 2737 and 1287 / 1299 / 1300 /
+ * 1336, hi + lo 1622 / 1702 / 2162 / 3152 and 1723 / 1736 / 1768 / 1862; box of
+ * 16384 points FP64 168 / 201 / 282 / 353 and 167 / 169 / 170 / 174, FP32 145 /
+ * 162 / 209 / 295 and 137 at any.  A stage of few segments in FP64 leaves the
+ * matrix cores waiting: curve of 5000 points 110 / 123 / 148 / 209 and 149 at
+ * any, so such a stage changes over at 8. */
+#define MFMA_LEAST_F64 6
+#define MFMA_LEAST_F64_SMALL 8 /* under MFMA_SMALL segments */
+#define MFMA_LEAST_F32 5
+#define MFMA_LEAST_F32X2 6
+#define MFMA_SMALL 4096
+static int mfma_stage(int nrhs, int cfg, int least) {
+  return nrhs >= 16 && cfg >= 0 ? cfg != 0 : nrhs >= least && g_mfmaCT != 0;
+}
+/* its launch shape: below 16 right-hand sides one column tile */
+static int mfma_shape(int nrhs, int cfg, int dflt) {
+  if (nrhs >= 16 && cfg >= 0) return cfg;
+  if (nrhs >= 16 && g_mfmaCT > 0) return g_mfmaCT;
+  return mfma_auto(g_mfmaCT > 0 ? g_mfmaCT : dflt, nrhs);
+}
+
 static int launch_stage_f64(const BfkSeg *segs, int64_t n, const BfkStageShape &shape, const BfkTerm *dTerms,
                             const double *dArena, const BfkBufs &b, int nrhs, int cfg) {
   if (n == 0) return 0;
-  if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
-    const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F64, nrhs);
+  if (mfma_stage(nrhs, cfg, n < MFMA_SMALL ? MFMA_LEAST_F64_SMALL : MFMA_LEAST_F64)) {
+    const int mc = mfma_shape(nrhs, cfg, MFMA_DEFAULT_F64);
     launch_mfma<MfmaF64, false, false>(mc, segs, shape, dTerms, (const double2 *)dArena, nullptr, b, nrhs, n);
     BFK_CHECK(hipGetLastError());
   } else {
@@ -3380,8 +3406,11 @@ static int launch_stage_f32(const BfkSeg *segs, int64_t n, const BfkStageShape &
                             const float *dArenaHi, const float *dArenaLo, const BfkBufsF &b, int nrhs, int cfg) {
   if (n == 0) return 0;
   const float2 *H = (const float2 *)dArenaHi, *Lo = (const float2 *)dArenaLo;
-  if (nrhs >= 16 && (cfg >= 0 ? cfg : g_mfmaCT != 0)) {
-    const int mc = cfg >= 0 ? cfg : g_mfmaCT > 0 ? g_mfmaCT : mfma_auto(MFMA_DEFAULT_F32, nrhs);
+  /* plain FP32 sums, where they are asked for, stay on the vector unit below
+   * 16: the matrix cores' are twice as far off */
+  const int least = Lo ? MFMA_LEAST_F32X2 : g_comp32 ? MFMA_LEAST_F32 : 16;
+  if (mfma_stage(nrhs, cfg, least)) {
+    const int mc = mfma_shape(nrhs, cfg, MFMA_DEFAULT_F32);
     if (Lo) { /* hi + lo summed in FP64 on load, the FP64 matrix cores */
       launch_mfma<MfmaF64S32, true, false>(mc, segs, shape, dTerms, H, Lo, b, nrhs, n);
     } else if (g_comp32 == 1) {

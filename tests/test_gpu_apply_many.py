@@ -26,7 +26,7 @@ def test_one_dense_block(gpu_lib, m, n):
     lib.bfMatBlockDiagInit(d, 1, 1)
     lib.bfMatBlockDiagSetBlock(d, 0, dense.ptr)
     P = gpu_lib.Mat(lib.bfhipMatPack(d))
-    for nrhs in (16, 17, 32, 33, 64, 130):
+    for nrhs in (5, 8, 15, 16, 17, 32, 33, 64, 130):
         X = rand(rng, n, nrhs)
         # each of n complex products and sums is off by at most a few 2^-53 of |A| |X|
         bound = 4 * n * 2.0 ** -52 * (np.abs(A) @ np.abs(X))
@@ -45,7 +45,7 @@ def test_many_columns_equal_one_column(gpu_lib, geometry, n, leaf):
     rng = np.random.default_rng(5)
     X = rng.standard_normal((n, 70)) + 1j * rng.standard_normal((n, 70))
     one = np.concatenate([apply(bf, F, X[:, c:c + 1], "fp64") for c in range(70)], 1)
-    many = (16, 19, 33, 70)
+    many = (5, 6, 7, 8, 11, 15, 16, 19, 33, 70)
     for nrhs in many:
         # the same products in another order: the sums of a stage have up to
         # 2000 terms, of 10 stages
