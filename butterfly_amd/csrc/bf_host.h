@@ -61,6 +61,8 @@ int bfk_scale_rows(int64_t n, int nrhs, const double *dW, const void *dX, void *
 int bfk_bie_post(int64_t n, int nrhs, int ncorr, double alpha, const int32_t *dCol, const double *dC,
                  const void *dX, const void *dU, void *dY, int fp32);
 int bfk_dotc_multi(int64_t n, int nv, const double *dV, int64_t ldv, const double *dW, double *hOut);
+int bfk_dotc_multi_dev(int64_t n, int nv, const double *dV, int64_t ldv, const double *dW, double *dH);
+int bfk_axpy_multi_dev(int64_t n, int nv, const double *dV, int64_t ldv, const double *dH, double s, double *dW);
 int bfk_axpy_multi(int64_t n, int nv, const double *dV, int64_t ldv, const double *hH, double s, double *dW);
 int bfk_convert(int64_t n, const void *src, void *dst, int to32);
 int bfk_svd_jacobi(int64_t nb, const int32_t *dIdx, const int64_t *dAOff, const int32_t *dM, const int32_t *dN,

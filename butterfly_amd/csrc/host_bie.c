@@ -227,6 +227,7 @@ typedef struct {
   int64_t n;
   int m;            /* Krylov dimension per cycle */
   double *dV;       /* (m + 1) x n, column j at dV + 2 j n */
+  double *dH;       /* the coefficients of one step: 2 (m + 1) + 1 complex */
   float *dv32, *dw32;
 } Gmres;
 
@@ -263,7 +264,7 @@ static int gmres_solve(Gmres *G, const double *db, double *dx, double tol, int m
   double *H = calloc((size_t)(m + 1) * m * 2, sizeof(double)); /* column-major (m+1) x m complex */
   double *cs = calloc((size_t)m, sizeof(double)), *sn = calloc((size_t)m * 2, sizeof(double));
   double *gv = calloc((size_t)(m + 1) * 2, sizeof(double));
-  double *h = calloc((size_t)(m + 1) * 2, sizeof(double)), *h2 = calloc((size_t)(m + 1) * 2, sizeof(double));
+  double *h = calloc((size_t)(m + 1) * 4 + 2, sizeof(double));
   double *y = calloc((size_t)m * 2, sizeof(double));
   double one[2] = {1, 0};
   int done = 0;
@@ -285,14 +286,17 @@ static int gmres_solve(Gmres *G, const double *db, double *dx, double tol, int m
     for (int j = 0; j < m && !rc && *iters < maxIter; ++j) {
       double *w = vcol(G, j + 1);
       rc = op_apply(G, vcol(G, j), w, fp32);
-      /* classical Gram-Schmidt, twice */
-      if (!rc) rc = bfk_dotc_multi(n, j + 1, G->dV, n, w, h);
-      if (!rc) rc = bfk_axpy_multi(n, j + 1, G->dV, n, h, 1.0, w);
-      if (!rc) rc = bfk_dotc_multi(n, j + 1, G->dV, n, w, h2);
-      if (!rc) rc = bfk_axpy_multi(n, j + 1, G->dV, n, h2, 1.0, w);
-      double hn = 0;
-      if (!rc) rc = dev_norm(G, w, &hn);
+      /* classical Gram-Schmidt, twice; the coefficients stay on the device
+       * until both and the norm are there: h, h2, |w|^2 in one download */
+      double *dh2 = G->dH + 2 * (j + 1), *dn = dh2 + 2 * (j + 1);
+      if (!rc) rc = bfk_dotc_multi_dev(n, j + 1, G->dV, n, w, G->dH);
+      if (!rc) rc = bfk_axpy_multi_dev(n, j + 1, G->dV, n, G->dH, 1.0, w);
+      if (!rc) rc = bfk_dotc_multi_dev(n, j + 1, G->dV, n, w, dh2);
+      if (!rc) rc = bfk_axpy_multi_dev(n, j + 1, G->dV, n, dh2, 1.0, w);
+      if (!rc) rc = bfk_dotc_multi_dev(n, 1, w, n, w, dn);
+      if (!rc) rc = bfk_d2h(h, G->dH, (size_t)(2 * (j + 1) + 1) * 16);
       if (rc) break;
+      const double *h2 = h + 2 * (j + 1), n2 = h2[2 * (j + 1)], hn = sqrt(n2 > 0 ? n2 : 0);
       for (int i = 0; i <= j; ++i) {
         H[2 * (j * (m + 1) + i)] = h[2 * i] + h2[2 * i];
         H[2 * (j * (m + 1) + i) + 1] = h[2 * i + 1] + h2[2 * i + 1];
@@ -366,7 +370,7 @@ static int gmres_solve(Gmres *G, const double *db, double *dx, double tol, int m
     for (int i = 0; i < k; ++i) { y[2 * i] = -y[2 * i]; y[2 * i + 1] = -y[2 * i + 1]; }
     rc = bfk_axpy_multi(n, k, G->dV, n, y, 1.0, dx); /* x += V y */
   }
-  free(H); free(cs); free(sn); free(gv); free(h); free(h2); free(y);
+  free(H); free(cs); free(sn); free(gv); free(h); free(y);
   return rc;
 }
 
@@ -376,7 +380,8 @@ static int gmres_init(Gmres *G, BfMatHipBie *A, int m, int fp32) {
   G->n = A->n;
   G->m = m;
   G->dV = bfk_malloc((size_t)(m + 1) * (size_t)A->n * 16);
-  if (!G->dV) return -2;
+  G->dH = bfk_malloc((size_t)(2 * m + 1) * 16);
+  if (!G->dV || !G->dH) return -2;
   if (fp32) {
     G->dv32 = bfk_malloc((size_t)A->n * 8);
     G->dw32 = bfk_malloc((size_t)A->n * 8);
@@ -387,6 +392,7 @@ static int gmres_init(Gmres *G, BfMatHipBie *A, int m, int fp32) {
 
 static void gmres_free(Gmres *G) {
   bfk_free(G->dV);
+  bfk_free(G->dH);
   bfk_free(G->dv32);
   bfk_free(G->dw32);
 }
