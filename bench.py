@@ -465,7 +465,7 @@ def main():
     # this kernel and workload, scaled by the counters' reading of a plain
     # copy (the summary file gives the commands)
     traffic = None
-    tpath = os.path.join(ROOT, "profiles", "k_apply1_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "k_apply_few_traffic.json")
     if n == 1 << 20 and args.tol == 1e-8 and args.rank_const == 1.25 and os.path.exists(tpath):
         traffic = json.load(open(tpath))["traffic_bytes_per_apply"]
 
@@ -657,7 +657,7 @@ def main():
         "dense_rows": args.rows,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "k_apply1 (all stages of one apply)", "bytes_per_apply": bytes_per_apply,
+                     "kernel": "k_apply_few (all stages of one apply)", "bytes_per_apply": bytes_per_apply,
                      "event_ms_per_apply": apply_ms},
         "mixed": mixed,
         "split": split,

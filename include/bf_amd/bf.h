@@ -493,7 +493,8 @@ void bfhipGetKernelTimeSums(double sums[8], double counts[8]);
 void bfhipResetKernelTimes(void);
 /* new: launch shapes of the apply, for tuning: the 1-RHS apply's waves per
  * block in {1, 2, 4} (one row segment per wave where segments are not split
- * over waves; `unroll` is accepted and has no effect: the lane map follows
+ * over waves; 5 to 15 right-hand sides run on the matrix cores where their
+ * 16 padded columns cost less, unless the tiles below are 0; `unroll` is accepted and has no effect: the lane map follows
  * the segment's height); the many-RHS apply's right-hand-side
  * tiles of 16 per wave on the matrix cores in {1, 2, 4, 8}, plus 16 for
  * two 16-row tiles per wave (tiles 1, 2 or 4), 0 for the vector-unit

@@ -1,0 +1,44 @@
+"""The batched SVD at the shapes where its path changes: QR in registers and
+in LDS, Jacobi of the triangle by a whole workgroup (up to 70 columns) and by
+blocks of 8 rows (71 to 256), each as is and transposed, several shapes in
+one batch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def graded(rng, m, n):
+    """sigma_0 = 1, exponents spread over 14 decades but none within a factor
+    of 10 of the cut 1e-7, where rounding would decide the rank"""
+    p = min(m, n)
+    u = np.linalg.qr(rng.standard_normal((m, p)) + 1j * rng.standard_normal((m, p)))[0]
+    v = np.linalg.qr(rng.standard_normal((n, p)) + 1j * rng.standard_normal((n, p)))[0]
+    e = 12 * rng.random(p)
+    e = np.where(e > 6, e + 2, e)
+    e[0] = 0
+    return (u * 10.0 ** -np.sort(e)) @ v.conj().T
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (2, 1), (16, 16), (17, 17), (33, 8), (70, 70), (71, 71), (72, 71), (255, 64),
+                                 (256, 64), (257, 64), (256, 65), (256, 70), (256, 71), (200, 150), (256, 256),
+                                 (512, 32), (512, 33), (513, 32), (700, 80)])
+def test_svd_at_the_edges_of_its_paths(gpu_lib, m, n):
+    rng = np.random.default_rng(1000 * m + n)
+    # the shape twice, transposed, rank 3 with a zero column, and a small one
+    mats = [graded(rng, m, n), graded(rng, m, n), graded(rng, n, m), graded(rng, 9, 5)]
+    r = min(3, m, n)
+    low = (rng.standard_normal((m, r)) + 1j * rng.standard_normal((m, r))) @ rng.standard_normal((r, n))
+    if n > 1:
+        low[:, n // 2] = 0
+    mats.append(low)
+    tol = 1e-7
+    for A, (U, W, k) in zip(mats, gpu_lib.svd_batched(mats, tol)):
+        s = np.linalg.svd(A, compute_uv=False)
+        assert k == int(np.sum(s >= tol * s[0]))
+        # each of ~10 sweeps of n rotations is off by a few 2^-53
+        eps = 2.0 ** -52 * max(m, n) * 40
+        assert np.abs(U.conj().T @ U - np.eye(k)).max() < eps
+        assert np.abs(np.linalg.norm(W, axis=1) - s[:k]).max() <= eps * s[0]
+        rest = s[k] if k < len(s) else 0
+        assert np.linalg.norm(U @ W - A, 2) <= rest * 1.0001 + eps * s[0]
