@@ -510,10 +510,10 @@ int bfhipSetApplyConfig(int wavesPerBlock, int unroll, int mfmaTiles);
  * many times (iterative solvers, batched serving). */
 int bfhipSetApplyGraphs(int on);
 /* new (no counterpart): waves per re-expansion block in the compression.
- * Blocks whose LDS workspace (4-KiB classes) exceeds `twoAbove` bytes are
- * solved by 2 waves, above `fourAbove` by 4 (defaults 16384 and 40960:
- * the p >~ 22 blocks, whose LDS leaves room for only a few per CU); the
- * others by one wave.  Every shape gives the reference's pseudo-inverse
+ * Blocks (one to four that invert the same matrix together) whose LDS
+ * workspace (4-KiB classes) exceeds `twoAbove` bytes are solved by 2 waves,
+ * above `fourAbove` by 4 (defaults 16384 and 40960: their LDS leaves room
+ * for only a few per CU); the others by one wave.  Every shape gives the reference's pseudo-inverse
  * solution; they differ only in the order of rounding.  A negative value
  * leaves that threshold unchanged; the previous values go to *oldTwo /
  * *oldFour when not NULL.  Applies to the factorizations made after the
