@@ -1955,7 +1955,8 @@ __device__ __forceinline__ void ortho_rmul(double2 *__restrict__ M, int ld, int 
  * by its row's R_in (upper triangular, in place, rows ascending), then for
  * rOut >= 0 a Householder QR of the stacked column: R goes to rOut and the
  * blocks are overwritten by the matching rows of Q, formed in place from
- * the reflectors (last reflector first). */
+ * the reflectors (last reflector first).  With rows < n there are `rows`
+ * reflectors, Q = [Q' | 0] and R = [R'; 0]. */
 __global__ __launch_bounds__(64) void k_ortho(const BfkOrthoJob *__restrict__ jobs, const int32_t *__restrict__ order,
                                               const BfkOrthoItem *__restrict__ items, double2 *__restrict__ arena,
                                               const double2 *__restrict__ rIn, double2 *__restrict__ rOut) {
@@ -1991,7 +1992,8 @@ __global__ __launch_bounds__(64) void k_ortho(const BfkOrthoJob *__restrict__ jo
 
   if (J.rOut >= 0) {
     /* Householder QR, reflector j: v = x + ph sig e_j, H = I - v v^H / (sig (sig + |x_j|)) */
-    for (int j = 0; j < n; ++j) {
+    const int kq = min(rows, n);
+    for (int j = 0; j < kq; ++j) {
       double s = 0;
       for (int r = j + lane; r < rows; r += 64) {
         double2 a = M[j * ld + r];
@@ -2016,17 +2018,17 @@ __global__ __launch_bounds__(64) void k_ortho(const BfkOrthoJob *__restrict__ jo
     double2 *Ro = rOut + J.rOut;
     for (int e = lane; e < n * n; e += 64) {
       const int c = e / n, r = e - c * n;
-      Ro[e] = r < c ? M[c * ld + r] : (r == c ? dg[c] : make_double2(0, 0));
+      Ro[e] = r >= kq || r > c ? make_double2(0, 0) : r < c ? M[c * ld + r] : dg[c];
     }
     __syncthreads();
-    for (int e = lane; e < n * n; e += 64) {
-      const int c = e / n, r = e - c * n;
+    for (int e = lane; e < kq * n; e += 64) {
+      const int c = e / kq, r = e - c * kq;
       if (r < c) M[c * ld + r] = make_double2(0, 0);
     }
     __syncthreads();
-    for (int j = n - 1; j >= 0; --j) {
+    for (int j = kq - 1; j >= 0; --j) {
       const double iv = inv[j];
-      if (iv != 0) ortho_reflect_any(M, ld, j, rows, n, iv);
+      if (iv != 0) ortho_reflect_any(M, ld, j, rows, kq, iv);
       __syncthreads();
       const double2 v0 = M[j * ld + j];
       __syncthreads();
