@@ -3086,7 +3086,7 @@ int bfk_svd_jacobi_big(int64_t nb, const int32_t *dBig, const int64_t *dAOff, co
                        dN, dVOff, (double2 *)dV);
     if (hipGetLastError() != hipSuccess) rc = -1;
   }
-  for (int sweep = 0; sweep < maxSweeps && !rc && P > 2; ++sweep) {
+  for (int sweep = 0; sweep < maxSweeps && !rc && maxN >= 2; ++sweep) {
     int any = 0;
     for (int64_t i = 0; i < nb; ++i) any |= act[i];
     if (!any) break;

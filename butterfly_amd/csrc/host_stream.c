@@ -259,6 +259,7 @@ typedef struct {
 
 static int svd_split(SvdSplit *p, int64_t nj, const int64_t *aOff, const int32_t *M, const int32_t *N) {
   memset(p, 0, sizeof(*p));
+  if (bfk_init()) return -1; /* the limits below are the device's */
   p->idx = malloc(nz(4 * nj) * sizeof(int32_t));
   if (!p->idx) return -2;
   const int limit[2] = {bfk_svd_tall_max_n(), bfk_svd_qr_max_n()};
@@ -270,12 +271,14 @@ static int svd_split(SvdSplit *p, int64_t nj, const int64_t *aOff, const int32_t
     if (N[i] > p->maxN[c]) p->maxN[c] = N[i];
     if (c < 2 && aOff[i] + e > p->end) p->end = aOff[i] + e;
   }
-  for (int c = 0; c < 4; ++c) p->chunk[c] = p->cnt[c] > 0 ? p->cnt[c] : 1;
+  for (int c = 0; c < 4; ++c) {
+    p->chunk[c] = p->cnt[c] > 0 ? p->cnt[c] : 1;
+    if (c < 3 && p->chunk[c] > 65535) p->chunk[c] = 65535; /* a grid's second dimension */
+  }
   for (int c = 0; c < 2; ++c) {
     if (!p->cnt[c]) continue;
     const int64_t most = (int64_t)(SVD_SCRATCH_MAX / bfk_svd_qr_scratch(1, p->maxN[c]));
     if (p->chunk[c] > most) p->chunk[c] = most;
-    if (p->chunk[c] > 65535) p->chunk[c] = 65535;
     const size_t b = bfk_svd_qr_scratch(p->chunk[c], p->maxN[c]);
     if (b > p->scratch) p->scratch = b;
   }

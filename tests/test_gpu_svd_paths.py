@@ -2,8 +2,14 @@
 in LDS, Jacobi of the triangle by a whole workgroup (up to 70 columns) and by
 blocks of 8 rows (71 to 256), each as is and transposed, several shapes in
 one batch."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
+
+from conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +48,29 @@ def test_svd_at_the_edges_of_its_paths(gpu_lib, m, n):
         assert np.abs(np.linalg.norm(W, axis=1) - s[:k]).max() <= eps * s[0]
         rest = s[k] if k < len(s) else 0
         assert np.linalg.norm(U @ W - A, 2) <= rest * 1.0001 + eps * s[0]
+
+
+FIRST = """
+import numpy as np
+import butterfly_amd as bf
+rng = np.random.default_rng(7)
+shapes = {shapes}
+mats = [rng.standard_normal(s) + 1j * rng.standard_normal(s) for s in shapes]
+first, second = bf.svd_batched(mats, 1e-7), bf.svd_batched(mats, 1e-7)
+for A, (U, W, k), (U2, W2, k2) in zip(mats, first, second):
+    assert k == k2 == min(A.shape) and np.array_equal(U, U2) and np.array_equal(W, W2), A.shape
+    eps = 2.0 ** -52 * max(A.shape) * 40
+    assert np.abs(U.conj().T @ U - np.eye(k)).max() < eps, A.shape
+    assert np.linalg.norm(U @ W - A, 2) < eps * np.linalg.norm(A, 2), A.shape
+print("same")
+"""
+
+
+@pytest.mark.parametrize("shapes", [[(40, 2), (2, 9), (5, 1)], [(60, 30), (200, 90), (3, 2), (12, 12)]])
+def test_svd_as_the_first_call_of_a_process(gpu_lib, shapes):
+    """A process whose first device call is a batched SVD takes the same path
+    as one that has used the device before, also where no matrix has more
+    than two columns."""
+    out = subprocess.run([sys.executable, "-c", FIRST.format(shapes=shapes)], cwd=ROOT, capture_output=True, text=True,
+                         timeout=100, env=dict(os.environ, PYTHONPATH=ROOT))
+    assert out.returncode == 0 and "same" in out.stdout, out.stdout + out.stderr
