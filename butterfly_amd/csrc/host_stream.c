@@ -195,10 +195,13 @@ static int cmp_sig_desc(const void *a, const void *b) {
 /* The workspace of a streamer's SVDs: device memory and page-locked host
  * memory for the copies, grown as needed and released with the streamer
  * (bounded by what its largest round takes).  A call without one makes its
- * own, in ordinary host memory. */
+ * own, in ordinary host memory, and so does a streamer that gets no
+ * page-locked memory; where the quarter to grow into does not fit, the
+ * workspace has the size asked for. */
 typedef struct {
   char *dev, *host;
   size_t devBytes, hostBytes;
+  int lock;   /* page-locked host memory is asked for */
   int locked; /* host is page-locked */
 } SvdWork;
 
@@ -207,21 +210,27 @@ static void svd_host_free(SvdWork *w) {
   else free(w->host);
   w->host = NULL;
   w->hostBytes = 0;
+  w->locked = 0;
 }
 
 static int svd_work(SvdWork *w, size_t dev, size_t host) {
   if (dev > w->devBytes) {
     bfk_free(w->dev);
     w->devBytes = 0;
-    w->dev = bfk_malloc(dev + dev / 4);
+    size_t n = dev + dev / 4;
+    w->dev = bfk_malloc(n);
+    if (!w->dev) w->dev = bfk_malloc(n = dev);
     if (!w->dev) return -2;
-    w->devBytes = dev + dev / 4;
+    w->devBytes = n;
   }
   if (host > w->hostBytes) {
     svd_host_free(w);
-    w->host = w->locked ? bfk_host_malloc(host + host / 4) : malloc(host);
+    size_t n = host + host / 4;
+    w->host = w->lock ? bfk_host_malloc(n) : NULL;
+    w->locked = w->host != NULL;
+    if (!w->host) w->host = malloc(n = host);
     if (!w->host) return -2;
-    w->hostBytes = w->locked ? host + host / 4 : host;
+    w->hostBytes = n;
   }
   return 0;
 }
@@ -950,7 +959,7 @@ void bfFacStreamerInit(BfFacStreamer *s, BfFacSpec const *spec) {
   s->ct = tree_view(spec->colTree);
   s->rowRevPerm = spec->rowTree->perm ? bfPermGetReversePerm(spec->rowTree->perm) : NULL;
   size_t nc = count_nodes(s->ct, 0);
-  s->rank.work.locked = 1;
+  s->rank.work.lock = 1;
   s->post = malloc(nc * sizeof(int32_t));
   s->numPost = 0;
   post_order(s->ct, 0, s->post, &s->numPost);
