@@ -1311,6 +1311,10 @@ __device__ __forceinline__ double house_apply_wave(const double2 *__restrict__ x
  * this takes 0.9, and 85 ms for 256 x 180 where this takes 3. */
 #define SVD_TALL_MAX_N 70
 #define SVD_QR_MAX_N 256
+/* The norm of a column from its square, 0 (no reflector) where a reflector's
+ * scale, about 1 / square, would be out of range: what the elimination leaves
+ * of a column's exact copies shrinks by 2^-52 a step and comes by there. */
+__device__ __forceinline__ double house_norm(double sq) { return sq > 1e-290 ? sqrt(sq) : 0.0; }
 #define SVD_TALL_T 1024 /* threads of the QR, Jacobi and W launches */
 __host__ __device__ __forceinline__ int tall_ld(int n) { return 2 * n + 1; }
 /* [R | I] and the reductions of 16 waves */
@@ -1366,7 +1370,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
     wave_argmax(best, bi);
     for (int o = 32; o > 0; o >>= 1) free1 = min(free1, __shfl_xor(free1, o, 64));
     const int p = __builtin_amdgcn_readfirstlane(bi < n ? bi : free1);
-    const double sg = sqrt(cn[p]);
+    const double sg = house_norm(cn[p]);
     if (w == (p & (NW - 1))) { /* the wave that holds it: the reflector */
 #pragma unroll
       for (int q = 0; q < CPW; ++q)
@@ -1523,7 +1527,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     }
     __syncthreads();
     double2 *x = s + (int64_t)j * m;
-    const double sg = sqrt(qnorm);
+    const double sg = house_norm(qnorm);
     const double2 x0 = x[j];
     const double ax0 = hypot(x0.x, x0.y);
     const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;
@@ -2000,7 +2004,7 @@ __global__ __launch_bounds__(64) void k_ortho(const BfkOrthoJob *__restrict__ jo
         s = fma(a.x, a.x, fma(a.y, a.y, s));
       }
       s = wave_sum(s);
-      const double sig = sqrt(s);
+      const double sig = house_norm(s);
       const double2 x0 = M[j * ld + j];
       const double ax0 = hypot(x0.x, x0.y);
       const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;

@@ -74,3 +74,19 @@ def test_svd_as_the_first_call_of_a_process(gpu_lib, shapes):
     out = subprocess.run([sys.executable, "-c", FIRST.format(shapes=shapes)], cwd=ROOT, capture_output=True, text=True,
                          timeout=100, env=dict(os.environ, PYTHONPATH=ROOT))
     assert out.returncode == 0 and "same" in out.stdout, out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-50, 1e-60])
+@pytest.mark.parametrize("m,copies", [(60, 24), (300, 24), (120, 40)])
+def test_svd_of_many_copies_of_two_columns(gpu_lib, scale, m, copies):
+    """What the elimination leaves of a column's copies shrinks by 2^-52 with
+    each step, down to numbers whose squares have no reciprocal."""
+    mats = []
+    for seed in range(30):
+        rng = np.random.default_rng(seed)
+        mats.append(scale * np.repeat(rng.standard_normal((m, 2)) + 1j * rng.standard_normal((m, 2)), copies, axis=1))
+    eps = 2.0 ** -52 * max(m, 2 * copies) * 40
+    for A, (U, W, k) in zip(mats, gpu_lib.svd_batched(mats, 1e-7)):
+        assert k == 2
+        assert np.abs(U.conj().T @ U - np.eye(2)).max() < eps
+        assert np.linalg.norm(U @ W - A, 2) <= eps * np.linalg.norm(A, 2)
