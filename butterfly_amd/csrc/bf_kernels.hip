@@ -357,6 +357,20 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return y;
 }
 
+/* a = |r_i|^2, b = |r_j|^2 and g = r_i . conj(r_j) of a pair of rows whose
+ * products leave the range: all three over |r_i| |r_j|, which leaves the
+ * rotation as it is */
+__device__ __forceinline__ void pair_range(double &a, double &b, double &gx, double &gy) {
+  const double ab = a * b;
+  if ((ab < 1e-250 || ab > 1e250) && a > 0 && b > 0) {
+    const double fa = 1.0 / sqrt(a), fb = 1.0 / sqrt(b);
+    a = a * fa * fb;
+    b = b * fa * fb;
+    gx = gx * fa * fb;
+    gy = gy * fa * fb;
+  }
+}
+
 /* One-sided Jacobi on the rows of R (p rows, W columns with the right-hand
  * part), round-robin pairs, LP lanes per pair (a power of two fixed at
  * compile time so the strides fold into the LDS offsets), on a workgroup
@@ -365,7 +379,8 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
  * rows i < j with g = r_i . conj(r_j), a = |r_i|^2, b = |r_j|^2:
  *   e = g/|g|, zeta = (b - a)/(2|g|), t = sign(zeta)/(|zeta| + sqrt(1 + zeta^2)),
  *   c = 1/sqrt(1 + t^2), s = c t;  r_i <- c r_i - s e r_j,  r_j <- s r_i + c e r_j.
- * With EXACT (the SVDs) sweeps go on until one rotates nothing. */
+ * With EXACT (the SVDs) sweeps go on until one rotates nothing, and rows of
+ * any norm are rotated. */
 template <int LP, int G, bool EXACT = false>
 __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int W, int ld, double *red) {
   const int lane = threadIdx.x;
@@ -419,8 +434,10 @@ __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int 
         be = group_sum(be, LP);
         gx = group_sum(gx, LP);
         gy = group_sum(gy, LP);
+        if (EXACT) pair_range(al, be, gx, gy);
         const double ag2 = gx * gx + gy * gy;
-        /* rows below 1e-145 in norm lie far under any cut; they are not rotated */
+        /* rows below 1e-145 in norm lie far under any cut; they are not rotated
+         * (without EXACT) */
         if (valid && ag2 > 1e-290 && ag2 > thr2 * al * be) {
           rotated = 1;
           big |= ag2 >= 1e-12 * (al * be);
@@ -1314,7 +1331,8 @@ __device__ __forceinline__ double house_apply_wave(const double2 *__restrict__ x
 /* The norm of a column from its square, 0 (no reflector) where a reflector's
  * scale, about 1 / square, would be out of range: what the elimination leaves
  * of a column's exact copies shrinks by 2^-52 a step and comes by there. */
-__device__ __forceinline__ double house_norm(double sq) { return sq > 1e-290 ? sqrt(sq) : 0.0; }
+#define HOUSE_LEAST 1e-290
+__device__ __forceinline__ double house_norm(double sq) { return sq > HOUSE_LEAST ? sqrt(sq) : 0.0; }
 #define SVD_TALL_T 1024 /* threads of the QR, Jacobi and W launches */
 __host__ __device__ __forceinline__ int tall_ld(int n) { return 2 * n + 1; }
 /* [R | I] and the reductions of 16 waves */
@@ -1357,6 +1375,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
   double2 diag[CPW]; /* the diagonal of R in the columns taken */
 #pragma unroll
   for (int q = 0; q < CPW; ++q) diag[q] = make_double2(0, 0);
+  int rank = n; /* rows of R from here on are zero */
   for (int j = 0; j < n; ++j) {
     /* the largest remaining column, the first among equals; where no
      * comparison holds (NaN) the first remaining one */
@@ -1371,6 +1390,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
     for (int o = 32; o > 0; o >>= 1) free1 = min(free1, __shfl_xor(free1, o, 64));
     const int p = __builtin_amdgcn_readfirstlane(bi < n ? bi : free1);
     const double sg = house_norm(cn[p]);
+    if (cn[p] <= HOUSE_LEAST) rank = min(rank, j); /* and with it what is left */
     if (w == (p & (NW - 1))) { /* the wave that holds it: the reflector */
 #pragma unroll
       for (int q = 0; q < CPW; ++q)
@@ -1438,7 +1458,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
 #pragma unroll
       for (int u = 0; u < RPL; ++u) {
         const int r = lane + 64 * u;
-        if (r < n) rg[r * ld + p] = r < p ? x[q][u] : r == p ? diag[q] : make_double2(0, 0);
+        if (r < n) rg[r * ld + p] = r >= rank || r > p ? make_double2(0, 0) : r < p ? x[q][u] : diag[q];
       }
     }
   }
@@ -1497,6 +1517,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     if (lane == 0) cn[c] = q;
   }
   __syncthreads();
+  int rank = n; /* rows of R from here on are zero */
   for (int j = 0; j < n; ++j) {
     if (w == 0) { /* the largest remaining column, the first among equals */
       double best = -1.0;
@@ -1528,6 +1549,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     __syncthreads();
     double2 *x = s + (int64_t)j * m;
     const double sg = house_norm(qnorm);
+    if (qnorm <= HOUSE_LEAST) rank = min(rank, j);
     const double2 x0 = x[j];
     const double ax0 = hypot(x0.x, x0.y);
     const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;
@@ -1557,7 +1579,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   for (int e = tid; e < n * 2 * n; e += SVD_TALL_T) {
     const int i = e / (2 * n), c = e - i * 2 * n;
     double2 v;
-    if (c < n) v = c > i ? s[(int64_t)c * m + i] : (c == i ? rdiag[i] : make_double2(0, 0));
+    if (c < n) v = i >= rank || c < i ? make_double2(0, 0) : c > i ? s[(int64_t)c * m + i] : rdiag[i];
     else v = make_double2(c - n == i ? 1.0 : 0.0, 0.0);
     rg[i * ld + c] = v;
   }
@@ -1646,6 +1668,7 @@ __global__ __launch_bounds__(SVD_BLK_T) void k_svd_block(const int32_t *__restri
       be = group_sum(be, 64);
       gx = group_sum(gx, 64);
       gy = group_sum(gy, 64);
+      pair_range(al, be, gx, gy);
       const double ag2 = gx * gx + gy * gy;
       if (ag2 > 1e-290 && ag2 > thr2 * al * be) { /* the rotation of jacobi_rows */
         rotated = 1;
@@ -1669,12 +1692,84 @@ __global__ __launch_bounds__(SVD_BLK_T) void k_svd_block(const int32_t *__restri
   for (int e = threadIdx.x; e < cj * ld; e += SVD_BLK_T) gj[e] = lj[e];
 }
 
-/* sigma and V of matrix t from [R' | G], a workgroup's threads over both.
- * A row that is exactly zero gets the unit vector of its pivot: the pivoted
- * QR leaves such rows last, for columns outside the others' span. */
+/* The columns of V that belong to rows of R' that are exactly zero (copies
+ * of columns, zero columns), here zero: each the unit vector that has most
+ * outside the span of the columns there are, made orthogonal to them twice.
+ * Rare, and seen only where nothing is cut off; w and h hold n entries, rem
+ * what is left of each unit vector (its square). */
+__device__ __forceinline__ void tall_complete_v(int n, const double *__restrict__ sgm, double2 *__restrict__ vo,
+                                                double2 *__restrict__ w, double2 *__restrict__ h,
+                                                double *__restrict__ rem) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int c = tid; c < n; c += SVD_TALL_T) {
+    double s = 1;
+    for (int k = 0; k < n; ++k) {
+      const double2 v = vo[(int64_t)k * n + c];
+      s -= v.x * v.x + v.y * v.y;
+    }
+    rem[c] = s;
+  }
+  __syncthreads();
+  for (int i = 0; i < n; ++i) {
+    if (!(sgm[i] == 0)) continue; /* uniform */
+    double best = -1e300;
+    int p = n;
+    for (int c = lane; c < n; c += 64)
+      if (rem[c] > best) { best = rem[c]; p = c; }
+    wave_argmax(best, p);
+    p = p < n ? p : 0; /* no comparison holds: NaN */
+    for (int c = tid; c < n; c += SVD_TALL_T) {
+      double2 a = make_double2(c == p ? 1.0 : 0.0, 0.0);
+      for (int k = 0; k < n; ++k) {
+        const double2 v = vo[(int64_t)k * n + c], q = vo[(int64_t)k * n + p]; /* minus v conj(q) */
+        a.x -= v.x * q.x + v.y * q.y;
+        a.y -= v.y * q.x - v.x * q.y;
+      }
+      w[c] = a;
+    }
+    __syncthreads();
+    for (int k = wave; k < n; k += SVD_TALL_T / 64) {
+      double sx = 0, sy = 0;
+      for (int c = lane; c < n; c += 64) {
+        const double2 v = vo[(int64_t)k * n + c], a = w[c]; /* conj(v) a */
+        sx = fma(v.x, a.x, fma(v.y, a.y, sx));
+        sy = fma(v.x, a.y, fma(-v.y, a.x, sy));
+      }
+      sx = group_sum(sx, 64);
+      sy = group_sum(sy, 64);
+      if (lane == 0) h[k] = make_double2(sx, sy);
+    }
+    __syncthreads();
+    for (int c = tid; c < n; c += SVD_TALL_T) {
+      double2 a = w[c];
+      for (int k = 0; k < n; ++k) {
+        const double2 v = vo[(int64_t)k * n + c], q = h[k];
+        a.x -= v.x * q.x - v.y * q.y;
+        a.y -= v.x * q.y + v.y * q.x;
+      }
+      w[c] = a;
+    }
+    __syncthreads();
+    double s = 0;
+    for (int c = lane; c < n; c += 64) s = fma(w[c].x, w[c].x, fma(w[c].y, w[c].y, s));
+    const double inv = 1.0 / sqrt(group_sum(s, 64));
+    for (int c = tid; c < n; c += SVD_TALL_T) {
+      const double2 a = make_double2(w[c].x * inv, w[c].y * inv);
+      vo[(int64_t)i * n + c] = a;
+      rem[c] -= a.x * a.x + a.y * a.y;
+    }
+    __syncthreads();
+  }
+}
+/* its scratch, in 16-byte units */
+__host__ __device__ __forceinline__ int tall_v_units(int n) { return 2 * n + (n + 1) / 2; }
+
+/* sigma and V of matrix t from [R' | G], a workgroup's threads over both;
+ * `work` holds tall_v_units(n) entries of LDS (2 n^2 hold them from n = 2 on,
+ * where the first column can be missing). */
 __device__ __forceinline__ void tall_sigma_v(const double2 *__restrict__ rg, int n, int ld, const int32_t *__restrict__ pv,
                                              double *__restrict__ sgm, double *__restrict__ sig,
-                                             double2 *__restrict__ vo) {
+                                             double2 *__restrict__ vo, double2 *__restrict__ work) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int i = w; i < n; i += SVD_TALL_T / 64) {
     double q = 0;
@@ -1690,9 +1785,19 @@ __device__ __forceinline__ void tall_sigma_v(const double2 *__restrict__ rg, int
     const int i = e / n, j = e - i * n;
     const double inv = sgm[i] > 0 ? 1.0 / sgm[i] : 0.0;
     const double2 r = rg[i * ld + j];
-    vo[(int64_t)i * n + pv[j]] =
-        sgm[i] > 0 ? make_double2(r.x * inv, -r.y * inv) : make_double2(sgm[i] == 0 && i == j ? 1.0 : 0.0, 0.0);
+    vo[(int64_t)i * n + pv[j]] = make_double2(r.x * inv, -r.y * inv);
   }
+  int zeros = 0;
+  for (int i = lane; i < n; i += 64) zeros += sgm[i] == 0;
+  for (int o = 32; o > 0; o >>= 1) zeros += __shfl_xor(zeros, o, 64);
+  if (zeros == 0) return; /* uniform over the workgroup */
+  __syncthreads();
+  if (zeros == n) { /* the zero matrix */
+    for (int i = tid; i < n; i += SVD_TALL_T) vo[(int64_t)i * n + i] = make_double2(1.0, 0.0);
+    __syncthreads();
+    return;
+  }
+  tall_complete_v(n, sgm, vo, work, work + n, (double *)(work + 2 * n));
 }
 
 __global__ __launch_bounds__(SVD_TALL_T) void k_tall_w(const int32_t *__restrict__ idx,
@@ -1714,7 +1819,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_w(const int32_t *__restrict
   const double *hinv = hinvg + (int64_t)t * maxN;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   constexpr int NW = SVD_TALL_T / 64;
-  tall_sigma_v(rg, n, ld, pv, sgm, sig + sOff[b], Vout + vOff[b]);
+  tall_sigma_v(rg, n, ld, pv, sgm, sig + sOff[b], Vout + vOff[b], lds);
   /* W = Q X, X = [sigma_c conj(G[c, :])^T; 0] (m x n, zero below row n),
    * Q = H_0 ... H_{n-1}, H_j = I - tau_j v_j v_j^H, v_j = column j of S on
    * rows >= j, tau_j = hinv[j] (0: no reflector).  Compact WY form:
@@ -1840,12 +1945,13 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_wide_w(const int32_t *__restrict
                                                        const int64_t *__restrict__ sOff, double *__restrict__ sig,
                                                        int maxN, int64_t slot) {
   __shared__ double sgm[SVD_QR_MAX_N];
+  __shared__ double2 work[2 * SVD_QR_MAX_N + SVD_QR_MAX_N / 2]; /* tall_v_units(SVD_QR_MAX_N) */
   const int t = blockIdx.y, b = idx[t];
   const int m = mm[b], n = nn[b], ld = tall_ld(n);
   const double2 *s = S + aOff[b], *rg = RG + (int64_t)t * slot;
   const double *hinv = hinvg + (int64_t)t * maxN;
   if (blockIdx.x == 0) {
-    tall_sigma_v(rg, n, ld, pivg + (int64_t)t * maxN, sgm, sig + sOff[b], Vout + vOff[b]);
+    tall_sigma_v(rg, n, ld, pivg + (int64_t)t * maxN, sgm, sig + sOff[b], Vout + vOff[b], work);
     return; /* the whole workgroup */
   }
   const int lane = threadIdx.x & 63, c = (int)(blockIdx.x - 1) * (SVD_TALL_T / 64) + (int)(threadIdx.x >> 6);

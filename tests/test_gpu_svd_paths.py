@@ -90,3 +90,40 @@ def test_svd_of_many_copies_of_two_columns(gpu_lib, scale, m, copies):
         assert k == 2
         assert np.abs(U.conj().T @ U - np.eye(2)).max() < eps
         assert np.linalg.norm(U @ W - A, 2) <= eps * np.linalg.norm(A, 2)
+        if scale < 1e-55:  # what rounding leaves is out of the column Jacobi's range (300 rows)
+            continue
+        U0, W0, k0 = gpu_lib.svd_batched([A.T], 0.0)[0]
+        assert k0 == min(A.shape)
+        assert np.abs(U0.conj().T @ U0 - np.eye(k0)).max() < eps
+        assert np.linalg.norm(U0 @ W0 - A.T, 2) <= eps * np.linalg.norm(A, 2)
+
+
+@pytest.mark.parametrize("m,n", [(6, 9), (21, 48), (48, 300), (60, 64), (90, 120), (96, 400)])
+def test_svd_of_repeated_rows_and_columns(gpu_lib, m, n):
+    """Exact copies leave exactly zero rows in the triangle: with no cut, the
+    vectors that belong to them are orthonormal to the others (U of a wide
+    matrix; a tall one's U has zero columns there)."""
+    rng = np.random.default_rng(m + n)
+    A = np.repeat(rng.standard_normal((m // 3, n)) + 1j * rng.standard_normal((m // 3, n)), 3, axis=0)
+    Z = np.zeros((m, n), complex)
+    Z[: m // 2] = rng.standard_normal((m // 2, n))
+    eps = 2.0 ** -52 * max(m, n) * 40
+    for B in (A, Z, np.zeros((m, n), complex)):
+        (U, W, k), (Ut, Wt, kt) = gpu_lib.svd_batched([B, B.T], 0.0)
+        assert k == kt == m
+        assert np.abs(U.conj().T @ U - np.eye(m)).max() < eps
+        assert np.linalg.norm(U @ W - B, 2) <= eps * np.linalg.norm(B, 2)
+        assert np.linalg.norm(Ut @ Wt - B.T, 2) <= eps * np.linalg.norm(B, 2)
+
+
+@pytest.mark.parametrize("scale", [1e-70, 1e70])
+@pytest.mark.parametrize("m,n", [(40, 12), (60, 60), (90, 200), (256, 250)])
+def test_svd_far_from_one(gpu_lib, scale, m, n):
+    """Entries whose fourth powers are out of range."""
+    A = scale * graded(np.random.default_rng(m), m, n)
+    U, W, k = gpu_lib.svd_batched([A], 1e-7)[0]
+    s = np.linalg.svd(A, compute_uv=False)
+    eps = 2.0 ** -52 * max(m, n) * 40
+    assert k == int(np.sum(s >= 1e-7 * s[0]))
+    assert np.abs(U.conj().T @ U - np.eye(k)).max() < eps
+    assert np.linalg.norm(U @ W - A, 2) <= (s[k] if k < len(s) else 0) * 1.0001 + eps * s[0]
