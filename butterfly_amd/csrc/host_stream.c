@@ -405,6 +405,11 @@ static int svd_batch(SvdJob *jobs, size_t nj, double tol, SvdWork *work) {
     qsort(si, (size_t)n, sizeof(SigIdx), cmp_sig_desc);
     int64_t k = 0; /* linalg.c:26-35 */
     while (k < n && si[k].s >= tol * si[0].s) ++k;
+    /* an entry that is not finite: rank 1 of NaN, so that what is made of
+     * the block shows it */
+    int bad = 0;
+    for (int64_t j = 0; j < n; ++j) bad |= !isfinite(s[j]);
+    if (bad) k = 1;
     J->k = k;
     J->truncated = k < n;
     /* for a block A = sum_j sigma_j u_j v_j^H (tall form):
@@ -414,7 +419,11 @@ static int svd_batch(SvdJob *jobs, size_t nj, double tol, SvdWork *work) {
     const int64_t Am = J->m, An = J->n;
     J->U = malloc((size_t)(Am * (k ? k : 1)) * sizeof(BfComplex));
     J->W = malloc((size_t)((k ? k : 1) * An) * sizeof(BfComplex));
-    for (int64_t q = 0; q < k; ++q) {
+    if (bad) {
+      for (int64_t r = 0; r < Am; ++r) J->U[r] = NAN;
+      for (int64_t c = 0; c < An; ++c) J->W[c] = NAN;
+    }
+    for (int64_t q = 0; q < k && !bad; ++q) {
       const int32_t j = si[q].j;
       const double sg = si[q].s;
       if (J->m >= J->n) {

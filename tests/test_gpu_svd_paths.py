@@ -127,3 +127,17 @@ def test_svd_far_from_one(gpu_lib, scale, m, n):
     assert k == int(np.sum(s >= 1e-7 * s[0]))
     assert np.abs(U.conj().T @ U - np.eye(k)).max() < eps
     assert np.linalg.norm(U @ W - A, 2) <= (s[k] if k < len(s) else 0) * 1.0001 + eps * s[0]
+
+
+@pytest.mark.parametrize("m,n", [(40, 12), (60, 60), (90, 200), (256, 250), (300, 50), (300, 260)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_svd_of_what_is_not_finite(gpu_lib, bad, m, n):
+    """It shows in the factors; its neighbours in the batch are not touched."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((m, n)) + 1j * rng.standard_normal((m, n))
+    B = A.copy()
+    B[3, 5] = bad
+    alone = gpu_lib.svd_batched([A], 1e-7)[0]
+    (U, W, k), beside = gpu_lib.svd_batched([B, A], 1e-7)
+    assert k > 0 and not np.isfinite(U @ W).all()
+    assert beside[2] == alone[2] and np.array_equal(beside[0], alone[0]) and np.array_equal(beside[1], alone[1])
