@@ -2192,7 +2192,8 @@ static int g_mfmaCT = -1;
 #define MFMA_SPLIT_TILE 4096
 /* A stage of few segments leaves the chip idle while each wave walks a long
  * chain.  Its row passes go to waves of their own while the segments (times
- * column chunks) number under 16384, two per wave slot in use; then, while
+ * column chunks) number under 16384, two per wave slot in use, or under 8192
+ * with two row tiles a wave, whose registers leave half the slots; then, while
  * there are fewer than 2048 such waves, 2 to 8 of them share the columns of
  * one pass (at least 8 steps of 4 each).  16 right-hand sides, one wave per
  * segment / row passes split / columns split too: 16 problems of 4096-65536
@@ -2202,13 +2203,30 @@ static int g_mfmaCT = -1;
  * 32768 and 65536 segments cost the curve of 100003 points 2.5 and 14% (a
  * segment's passes share its inputs in L1), the columns split at 4096 waves
  * the box 8%. */
+/* Waves for the passes of the tallest segment as long as all segments
+ * together make up to 16384 with it; otherwise for one and a half times the
+ * passes there are, so that a few tall segments don't make every other one
+ * launch waves that find nothing to do (a wave takes every rowGroups-th
+ * pass).  us with FP64 factors of curves, waves for the tallest everywhere /
+ * this rule: 40 right-hand sides at 8000 points 566 / 517, at 12000 901 / 744,
+ * 24 at 30000 1030 / 825, at 5000 40 take 325 / 366. */
 static int mfma_row_groups(int64_t numSegs, const BfkStageShape &sh, int chunks, int rowTiles) {
-  return numSegs * chunks < 16384 ? (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles) : 1;
+  const int64_t n = numSegs * chunks;
+  if (n >= 16384 / rowTiles) return 1;
+  int64_t g = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
+  if (n * g > 16384) {
+    const int64_t fit = (3 * sh.passes[rowTiles - 1] + 2 * numSegs - 1) / (2 * numSegs);
+    if (g > fit) g = fit;
+    if (n * g > (1 << 20)) g = (1 << 20) / n; /* a grid has less than 2^32 threads */
+  }
+  return (int)g;
 }
-static int mfma_split(int64_t numSegs, const BfkStageShape &sh, int items, int tiles) {
+static int mfma_split(int64_t numSegs, const BfkStageShape &sh, int items, int ct, int rowTiles) {
+  const int tiles = ct * rowTiles;
+  if (ct > 2) return 1; /* not built */
   const int64_t steps = numSegs > 0 ? sh.cols / numSegs / 4 : 0;
   int w = 1;
-  while (tiles <= 4 && w < MFMA_SPLIT_MAX && w * tiles < 16 && numSegs * items * w < 2048 && steps >= 16 * w) w *= 2;
+  while (w < MFMA_SPLIT_MAX && w * tiles < 16 && numSegs * items * w < 2048 && steps >= 16 * w) w *= 2;
   return w;
 }
 /* the default shape with no more column tiles than nrhs fills */
@@ -2572,7 +2590,7 @@ static void launch_mfma(int cfg, const BfkSeg *segs, const BfkStageShape &shape,
   const int chunks = (nrhs + 16 * ct - 1) / (16 * ct);
   const int groups = mfma_row_groups(numSegs, shape, chunks, rts);
   const dim3 grid(mfma_grid(numSegs, chunks * groups));
-  const int w = mfma_split(numSegs, shape, chunks * groups, rts * ct);
+  const int w = mfma_split(numSegs, shape, chunks * groups, ct, rts);
 #define BFK_MFMA_LAUNCH1(C, R)                                                                                       \
   hipLaunchKernelGGL((k_applyN_mfma<M, C, R, LO, COMP, false>), grid, dim3(64), 0, g_stream, segs, terms, H, Lo, b, \
                      nrhs, chunks, groups, numSegs)

@@ -34,6 +34,29 @@ def test_one_dense_block(gpu_lib, m, n):
     lib.bfMatDelete(C.byref(C.c_void_p(d)))
 
 
+# many short segments beside a tall one: the waves that the tall one's passes
+# get are bounded by the passes of all (one wave per pass in every segment
+# would be 4e9 threads and more at the second size)
+@pytest.mark.parametrize("short,m,nrhs", [(300, 20000, 40), (16000, 300000, 16), (3000, 33, 16)])
+def test_one_tall_block_among_short_ones(gpu_lib, short, m, nrhs):
+    lib = L()
+    rng = np.random.default_rng(m)
+    blocks = [rand(rng, 1 + i % 3, 2) for i in range(short)]
+    blocks.insert(short // 2, rand(rng, m, 3))
+    dense, d = [Dense(A) for A in blocks], lib.bfMatBlockDiagNew()
+    lib.bfMatBlockDiagInit(d, len(dense), len(dense))
+    for i, D in enumerate(dense):
+        lib.bfMatBlockDiagSetBlock(d, i, D.ptr)
+    P = gpu_lib.Mat(lib.bfhipMatPack(d))
+    X = rand(rng, 2 * short + 3, nrhs)
+    cols = np.cumsum([0] + [A.shape[1] for A in blocks])
+    want = np.concatenate([A @ X[c:c + A.shape[1]] for A, c in zip(blocks, cols)])
+    bound = np.concatenate([np.abs(A) @ np.abs(X[c:c + A.shape[1]]) for A, c in zip(blocks, cols)])
+    # at most three products and their sum, each off by a few 2^-53
+    assert (np.abs(P @ X - want) <= 12 * 2.0 ** -52 * bound).all()
+    lib.bfMatDelete(C.byref(C.c_void_p(d)))
+
+
 @pytest.mark.parametrize("geometry,n,leaf", [("curve", 4099, 64), ("box", 3001, 1)])
 def test_many_columns_equal_one_column(gpu_lib, geometry, n, leaf):
     bf = gpu_lib
