@@ -84,3 +84,31 @@ def test_many_columns_equal_one_column(gpu_lib, geometry, n, leaf):
                     assert rel(apply(bf, F, X[:, :nrhs], prec), one[:, :nrhs]) < (1e-6 if comp else 5e-6), (prec, comp)
             finally:
                 bf.lib().bfhipSetApplyCompensation(2)
+
+
+@pytest.mark.parametrize("comp", [3, 5, 9])
+def test_split_stages_with_coarser_folds(gpu_lib, comp):
+    """FP32 tiles folded into the FP64 sums every 2, 4 or 8 steps, in stages
+    whose columns are split over waves: the last of a curve (about 130
+    segments of 2000 columns, no multiple of 8 steps times the waves) and a
+    small box's.  A tile that a wave left unfolded would cost a share of the
+    columns, 1e-2 and more."""
+    bf = gpu_lib
+    for (src, tgt, k), leaf in ((curve_problem(4099), 64), (box_problem(1500), 32)):
+        n = len(src)
+        ts, tt = bf.Quadtree(src, leaf), bf.Quadtree(tgt, leaf)
+        F = bf.FacHelm2.make_multilevel(bf.Helm2(k), ts, tt,
+                                        bf.options(tol=1e-8, rank_const=1.25, pass_through=True, pinv_rcond=1e-11))
+        F.orthogonalize()
+        rng = np.random.default_rng(6)
+        X = rng.standard_normal((n, 37)) + 1j * rng.standard_normal((n, 37))
+        one = np.concatenate([apply(bf, F, X[:, c:c + 1], "fp64") for c in range(37)], 1)
+        F.prepare_mixed("fp32")
+        bf.lib().bfhipSetApplyCompensation(comp)
+        try:
+            for nrhs in (5, 16, 19, 37):
+                # FP32 vectors between ten stages, sums of 32 columns in FP32:
+                # 6e-8 each, times the root of 10 x (1 + 32 / 4)
+                assert rel(apply(bf, F, X[:, :nrhs], "fp32"), one[:, :nrhs]) < 1e-6, nrhs
+        finally:
+            bf.lib().bfhipSetApplyCompensation(2)
