@@ -1487,7 +1487,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   constexpr int NW = SVD_TALL_T / 64;
   {
-    __shared__ double2 vbuf[513]; /* the reflector and its scale */
+    __shared__ double2 vbuf[257]; /* the reflector and its scale */
     double2 *rg = RG + (int64_t)t * slot;
     int32_t *piv = pivg + (int64_t)t * maxN;
     double *hinv = hinvg + (int64_t)t * maxN;
@@ -1496,10 +1496,6 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     if (m <= 256 && n <= 64) {
       if (n <= 32) QR_REGS(4, 2);
       else QR_REGS(4, 4);
-      return;
-    }
-    if (m <= 512 && n <= 32) {
-      QR_REGS(8, 2);
       return;
     }
 #undef QR_REGS

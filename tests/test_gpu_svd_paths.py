@@ -1,7 +1,9 @@
-"""The batched SVD at the shapes where its path changes: QR in registers and
-in LDS, Jacobi of the triangle by a whole workgroup (up to 70 columns) and by
-blocks of 8 rows (71 to 256), each as is and transposed, several shapes in
-one batch."""
+"""The batched SVD at the shapes where its path changes: QR in registers (up to
+256 rows and 32 or 64 columns) and in global memory, Jacobi of the triangle by
+a whole workgroup (up to 70 columns) and by blocks of 8 rows (71 to 256), of
+the columns over the whole chip (from 257), and by one workgroup (more than
+256 rows, less than 2^15 entries), each as is and transposed, several shapes
+in one batch; and at the inputs where one of them could go wrong."""
 import os
 import subprocess
 import sys
@@ -28,7 +30,8 @@ def graded(rng, m, n):
 
 @pytest.mark.parametrize("m,n", [(1, 1), (2, 1), (16, 16), (17, 17), (33, 8), (70, 70), (71, 71), (72, 71), (255, 64),
                                  (256, 64), (257, 64), (256, 65), (256, 70), (256, 71), (200, 150), (256, 256),
-                                 (512, 32), (512, 33), (513, 32), (700, 80)])
+                                 (512, 32), (512, 33), (513, 32), (700, 80), (256, 32), (256, 33), (481, 68),
+                                 (482, 68), (469, 70), (462, 71), (300, 256), (257, 257), (300, 257)])
 def test_svd_at_the_edges_of_its_paths(gpu_lib, m, n):
     rng = np.random.default_rng(1000 * m + n)
     # the shape twice, transposed, rank 3 with a zero column, and a small one
