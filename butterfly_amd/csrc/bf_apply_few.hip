@@ -1,6 +1,7 @@
 /*
  * One stage of the apply on the vector units: one right-hand side and a few
- * (the many go to the matrix cores, k_applyN_mfma).
+ * (from 5 to 8 on, by type and stage size, the matrix cores take over,
+ * k_applyN_mfma).
  *
  * Bound: HBM, every stored factor entry is read once (16 B in FP64) and
  * meets NR right-hand sides in registers; what the shape of the kernel is
@@ -16,8 +17,8 @@
  *    One right-hand side in FP64 at 2^20 points: 12.1 ms, 6.2 TB/s of
  *    factors and vectors, what a plain read reaches here, in processes where
  *    the kernel before this one took 12.7 ms, and 13.7 ms in those where it
- *    took 14.5; FP32 at 2^19: 4.5 -> 3.4 ms; six right-hand sides at 100003
- *    points, before one lane a right-hand side: 37 -> 2.0 ms.
+ *    took 14.5; FP32 at 2^19: 4.5 -> 3.4 ms; four right-hand sides at 100003
+ *    points, before one lane a right-hand side: 37 -> 1.53 ms.
  *  - The columns of all terms are one sequence of steps, kept in a ring of
  *    RING steps in registers: the loads of the next RING - 1 steps are in
  *    flight while a step is multiplied, across term boundaries.  The terms
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * split_max(NR) : 256) void k_apply_few(
         /* the sums over the lanes, as far as there are terms: most segments
          * have one or two, and each of the six steps of a whole wave's scan
          * costs an LDS round trip (3 right-hand sides on 30000 points 401 ->
-         * 386 us, 6 on 100003 1950 -> 1920 us, box of 16384 points 123 -> 120 us) */
+         * 386 us, box of 16384 points 123 -> 120 us) */
         for (int d = 1; d < nT; d <<= 1) {
           const int o = __shfl_up(sum, d, 64);
           if (lane >= d) sum += o;

@@ -3556,9 +3556,9 @@ __global__ void k_to_f32(const double2 *__restrict__ a, int64_t n, float2 *__res
 extern "C" {
 
 /* accumulation of the FP32 applies: 0 plain FP32; 1 FP64 sums -- the
- * one-RHS kernel sums FP32 products in FP64, the matrix-core kernel widens
- * its FP32 operands and runs the FP64 matrix cores; 2 + mask (2 is the
- * default) the one-RHS kernel as 1, the matrix-core kernel accumulates
+ * vector-unit kernel widens its FP32 operands and multiplies and sums in
+ * FP64, the matrix-core kernel widens them and runs the FP64 matrix cores;
+ * 2 + mask (2 is the default) the vector-unit kernel as 1, the matrix-core kernel accumulates
  * FP32 tiles and folds them into FP64 sums every (mask + 1) 4-column steps
  * (mask 0, 1, 3 or 7) */
 int bfk_set_compensation(int on) {

@@ -1320,7 +1320,9 @@ int bfhipFacTuneApply(BfMat *fac, BfSize nrhs, BfhipPrecision prec, char const *
     return -1;
   }
   const int cls = bf_nrhs_class(nrhs);
-  if (cls == 1) return 0; /* 2-15 right-hand sides: the vector-unit kernel only */
+  /* 2-15 right-hand sides: nothing to choose, the vector unit or one column
+   * tile on the matrix cores by a fixed rule */
+  if (cls == 1) return 0;
   if (!cachePath) cachePath = getenv("BF_AMD_TUNE_CACHE");
   /* candidates: segments per block (1 RHS); tiles per MFMA wave x one or
    * two row tiles, 0 = the vector-unit kernel (16 and more) */

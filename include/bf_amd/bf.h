@@ -537,14 +537,13 @@ int bfhipFacTuneApply(BfMat *fac, BfSize nrhs, BfhipPrecision prec, char const *
 int bfhipFacGetApplyConfig(BfMat const *fac, BfSize nrhs, BfhipPrecision prec, int32_t *stageCfg);
 
 /* new: accumulation in the FP32 applies (factors and vectors stored in
- * FP32).  0: FP32 throughout.  1: FP64 sums -- one RHS: FP32 products
- * summed in FP64; many RHS: the FP32 operands widened to FP64 on load and
- * multiplied on the FP64 matrix cores -- so the rounding of a stage is one
- * FP32 rounding of its output however long its rows are.  2 + m (m = 0, 1,
- * 3 or 7): one RHS as 1; many RHS accumulate FP32 matrix-core tiles and
- * fold them into FP64 sums every m + 1 four-column steps.  The default is
- * 2 (a fold every step): at N = 2^20 and 256 RHS it is 1.13x faster than 1
- * at 8.6e-7 instead of 3.9e-7 relative error. */
+ * FP32).  0: FP32 throughout.  1: FP64 products and sums of the FP32
+ * operands, on the vector unit (one to four RHS) or the FP64 matrix cores,
+ * so the rounding of a stage is one FP32 rounding of its output however
+ * long its rows are.  2 + m (m = 0, 1, 3 or 7): on the vector unit as 1; on
+ * the matrix cores FP32 tiles folded into FP64 sums every m + 1 four-column
+ * steps.  The default is 2 (a fold every step): at N = 2^20 and 256 RHS it
+ * is 1.12x faster than 1 at 2.3e-7 instead of 1.3e-7 relative error. */
 int bfhipSetApplyCompensation(int on);
 
 /* new: plan export for parity checks (integers, in the oracle's canonical
