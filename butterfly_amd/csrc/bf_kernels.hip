@@ -2188,8 +2188,7 @@ static int g_mfmaCT = -1;
 #define MFMA_SPLIT_TILE 4096
 /* A stage of few segments leaves the chip idle while each wave walks a long
  * chain.  Its row passes go to waves of their own while the segments (times
- * column chunks) number under 16384, two per wave slot in use, or under 8192
- * with two row tiles a wave, whose registers leave half the slots; then, while
+ * column chunks) number under 16384, two per wave slot in use; then, while
  * there are fewer than 2048 such waves, 2 to 8 of them share the columns of
  * one pass (at least 8 steps of 4 each).  16 right-hand sides, one wave per
  * segment / row passes split / columns split too: 16 problems of 4096-65536
@@ -2199,22 +2198,29 @@ static int g_mfmaCT = -1;
  * 32768 and 65536 segments cost the curve of 100003 points 2.5 and 14% (a
  * segment's passes share its inputs in L1), the columns split at 4096 waves
  * the box 8%. */
-/* Waves for the passes of the tallest segment as long as all segments
- * together make up to 16384 with it; otherwise for one and a half times the
- * passes there are, so that a few tall segments don't make every other one
- * launch waves that find nothing to do (a wave takes every rowGroups-th
- * pass).  us with FP64 factors of curves, waves for the tallest everywhere /
- * this rule: 40 right-hand sides at 8000 points 566 / 517, at 12000 901 / 744,
- * 24 at 30000 1030 / 825, at 5000 40 take 325 / 366. */
+/* Waves for one and a half times the passes there are (a wave takes every
+ * rowGroups-th pass), so that a few tall segments don't make every other one
+ * launch waves that find nothing to do; but for all passes of a tallest
+ * segment far above the mean, whose chain would be the stage's time, as long
+ * as that makes no more than 2^17 waves.  With two row tiles a wave most
+ * segments are one pass, and the groups end at 4096 waves.  us of single
+ * stages in FP64, 40 right-hand sides, one wave per segment / one and a half
+ * per pass / one for each of the tallest's passes: 3770 segments, tallest 250
+ * rows, 198 / 152 / 109; 2168 segments, 195 rows, 120 / 94 / 55; 6098 segments,
+ * 64 rows, 73 / 103 / 103; FP32, 3310 segments, 58 rows, 124 / 62 / 72.  Whole
+ * applies with 16 to 80 right-hand sides on curves of 4096 to 20000 points are
+ * 4% faster than with waves for the tallest everywhere, and none is more than
+ * 3% slower. */
 static int mfma_row_groups(int64_t numSegs, const BfkStageShape &sh, int chunks, int rowTiles) {
-  const int64_t n = numSegs * chunks;
-  if (n >= 16384 / rowTiles) return 1;
-  int64_t g = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
-  if (n * g > 16384) {
-    const int64_t fit = (3 * sh.passes[rowTiles - 1] + 2 * numSegs - 1) / (2 * numSegs);
-    if (g > fit) g = fit;
-    if (n * g > (1 << 20)) g = (1 << 20) / n; /* a grid has less than 2^32 threads */
-  }
+  const int64_t n = numSegs * chunks, passes = sh.passes[rowTiles - 1];
+  if (n >= 16384) return 1;
+  const int64_t most = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
+  /* the tallest against the mean: 2.5 times while the chip has room, or 4 */
+  if (2 * most * numSegs >= (n * most <= 1 << 14 ? 5 : 8) * passes && n * most <= 1 << 17) return (int)most;
+  if (rowTiles == 2 && n >= 4096) return 1;
+  int64_t g = (3 * passes + 2 * numSegs - 1) / (2 * numSegs);
+  if (g > most) g = most;
+  if (n * g > 1 << 20) g = (1 << 20) / n; /* a grid has less than 2^32 threads */
   return (int)g;
 }
 static int mfma_split(int64_t numSegs, const BfkStageShape &sh, int items, int ct, int rowTiles) {
