@@ -2194,34 +2194,17 @@ static int g_mfmaCT = -1;
  * segment / row passes split / columns split too: 16 problems of 4096-65536
  * points in FP32 1187 / 1087 / 1087 us, box of 16384 points FP64 219 / 201 /
  * 198 us, FP32 183 / 145 / 145 us; curve of 4096 points FP32 236 / 127 / 108
- * us, of 5000 points with 20 in FP64 374 / 266 / 242 us.  Row passes split at
- * 32768 and 65536 segments cost the curve of 100003 points 2.5 and 14% (a
- * segment's passes share its inputs in L1), the columns split at 4096 waves
- * the box 8%. */
-/* Waves for one and a half times the passes there are (a wave takes every
- * rowGroups-th pass), so that a few tall segments don't make every other one
- * launch waves that find nothing to do; but for all passes of a tallest
- * segment far above the mean, whose chain would be the stage's time, as long
- * as that makes no more than 2^17 waves.  With two row tiles a wave most
- * segments are one pass, and the groups end at 4096 waves.  us of single
- * stages in FP64, 40 right-hand sides, one wave per segment / one and a half
- * per pass / one for each of the tallest's passes: 3770 segments, tallest 250
- * rows, 198 / 152 / 109; 2168 segments, 195 rows, 120 / 94 / 55; 6098 segments,
- * 64 rows, 73 / 103 / 103; FP32, 3310 segments, 58 rows, 124 / 62 / 72.  Whole
- * applies with 16 to 80 right-hand sides on curves of 4096 to 20000 points are
- * 4% faster than with waves for the tallest everywhere, and none is more than
- * 3% slower. */
+ * us, of 5000 points with 20 in FP64 374 / 266 / 242 us.  Row passes split up
+ * to 32768 or 65536 segments change applies of 12000 to 100003 points by -8 to
+ * 2% in the mixed forms and by -3 to 4% in FP64; the columns split at 4096
+ * waves cost the box 8%. */
+/* A wave for each pass of the tallest segment, in every segment (a wave takes
+ * every rowGroups-th pass): those that find no pass cost about a nanosecond
+ * each, the tallest's chain in fewer waves more. */
 static int mfma_row_groups(int64_t numSegs, const BfkStageShape &sh, int chunks, int rowTiles) {
-  const int64_t n = numSegs * chunks, passes = sh.passes[rowTiles - 1];
+  const int64_t n = numSegs * chunks, most = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
   if (n >= 16384) return 1;
-  const int64_t most = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
-  /* the tallest against the mean: 2.5 times while the chip has room, or 4 */
-  if (2 * most * numSegs >= (n * most <= 1 << 14 ? 5 : 8) * passes && n * most <= 1 << 17) return (int)most;
-  if (rowTiles == 2 && n >= 4096) return 1;
-  int64_t g = (3 * passes + 2 * numSegs - 1) / (2 * numSegs);
-  if (g > most) g = most;
-  if (n * g > 1 << 20) g = (1 << 20) / n; /* a grid has less than 2^32 threads */
-  return (int)g;
+  return (int)(n * most <= 1 << 20 ? most : (1 << 20) / n); /* a grid has less than 2^32 threads */
 }
 static int mfma_split(int64_t numSegs, const BfkStageShape &sh, int items, int ct, int rowTiles) {
   const int tiles = ct * rowTiles;
@@ -2335,15 +2318,21 @@ __global__ __launch_bounds__(SPLIT ? 64 * MFMA_SPLIT_MAX : 64) void k_applyN_mfm
    * b % 8 share an XCD (and its L2).  A group of MFMA_SEG_GROUP adjacent
    * segments (rows that read the same input blocks) with all their column
    * chunks gets the ids 8 * slot + xcd, so both the blocks and the inputs
-   * they share are read from one L2. */
+   * they share are read from one L2.  The row groups of its segments come one
+   * after another: the slots of an XCD go round its shader engines, and with a
+   * segment's row groups side by side the groups that few segments have (the
+   * second of two, the fourth of four) would all fall to the same engines and
+   * leave them idle (9558 segments of two passes, tallest six, FP32: 1 / 3 / 4 /
+   * 6 groups 74 / 55 / 86 / 58 us side by side, 76 / 56 / 56 / 58 so). */
   const int64_t slot = blockIdx.x >> 3;
   const int items = numChunks * rowGroups;
   const int64_t per = (int64_t)MFMA_SEG_GROUP * items;
   const int64_t grp = slot / per;
   const int64_t within = slot - grp * per;
-  const int64_t si = (grp * 8 + (blockIdx.x & 7)) * MFMA_SEG_GROUP + within / items;
-  const int item = (int)(within - (within / items) * items);
-  const int rowGroup = item / numChunks, chunk = item - rowGroup * numChunks;
+  const int groupItems = MFMA_SEG_GROUP * numChunks;
+  const int rowGroup = (int)(within / groupItems), item = (int)within - rowGroup * groupItems;
+  const int64_t si = (grp * 8 + (blockIdx.x & 7)) * MFMA_SEG_GROUP + item / numChunks;
+  const int chunk = item % numChunks;
   if (si >= numSegs) return;
   const BfkSeg Sg = segs[si];
   const int l = threadIdx.x & 63;

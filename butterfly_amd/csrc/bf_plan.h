@@ -81,11 +81,10 @@ typedef struct BfkTerm {
   int32_t xbuf;
 } BfkTerm;
 
-/* What the launch of a stage goes by: the columns of its terms and the passes
- * of 16 and of 32 rows, both summed over its segments, and the height of its
- * tallest segment. */
+/* What the launch of a stage goes by: the columns of its terms summed over
+ * its segments, and the height of its tallest segment. */
 typedef struct BfkStageShape {
-  int64_t cols, passes[2];
+  int64_t cols;
   int32_t maxRows, pad;
 } BfkStageShape;
 

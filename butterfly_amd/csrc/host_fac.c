@@ -127,8 +127,6 @@ BfkStageShape *bfStageShapes(const BfkSeg *segs, const int64_t *stageSeg, int nu
   for (int s = 0; s < numStages; ++s)
     for (int64_t i = stageSeg[s]; i < stageSeg[s + 1]; ++i) {
       if (segs[i].m > sh[s].maxRows) sh[s].maxRows = segs[i].m;
-      sh[s].passes[0] += (segs[i].m + 15) / 16;
-      sh[s].passes[1] += (segs[i].m + 31) / 32;
       for (int32_t t = segs[i].t0; t < segs[i].t1; ++t)
         if (terms[t].aOff >= 0) sh[s].cols += terms[t].n;
     }
