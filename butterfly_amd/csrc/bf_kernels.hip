@@ -357,18 +357,18 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return y;
 }
 
-/* a = |r_i|^2, b = |r_j|^2 and g = r_i . conj(r_j) of a pair of rows whose
- * products leave the range: all three over |r_i| |r_j|, which leaves the
- * rotation as it is */
-__device__ __forceinline__ void pair_range(double &a, double &b, double &gx, double &gy) {
+/* a = |r_i|^2, b = |r_j|^2 and g = r_i . conj(r_j) of a pair of rows that
+ * seems orthogonal: whether it is only that the products leave the range, and
+ * then all three over |r_i| |r_j|, which leaves the rotation as it is */
+__device__ __forceinline__ bool pair_range(double &a, double &b, double &gx, double &gy) {
   const double ab = a * b;
-  if ((ab < 1e-250 || ab > 1e250) && a > 0 && b > 0) {
-    const double fa = 1.0 / sqrt(a), fb = 1.0 / sqrt(b);
-    a = a * fa * fb;
-    b = b * fa * fb;
-    gx = gx * fa * fb;
-    gy = gy * fa * fb;
-  }
+  if (!((ab < 1e-250 || ab > 1e250) && a > 0 && b > 0)) return false;
+  const double fa = 1.0 / sqrt(a), fb = 1.0 / sqrt(b);
+  a = a * fa * fb;
+  b = b * fa * fb;
+  gx = gx * fa * fb;
+  gy = gy * fa * fb;
+  return true;
 }
 
 /* One-sided Jacobi on the rows of R (p rows, W columns with the right-hand
@@ -379,9 +379,9 @@ __device__ __forceinline__ void pair_range(double &a, double &b, double &gx, dou
  * rows i < j with g = r_i . conj(r_j), a = |r_i|^2, b = |r_j|^2:
  *   e = g/|g|, zeta = (b - a)/(2|g|), t = sign(zeta)/(|zeta| + sqrt(1 + zeta^2)),
  *   c = 1/sqrt(1 + t^2), s = c t;  r_i <- c r_i - s e r_j,  r_j <- s r_i + c e r_j.
- * With EXACT (the SVDs) sweeps go on until one rotates nothing, and rows of
- * any norm are rotated. */
-template <int LP, int G, bool EXACT = false>
+ * With EXACT (the SVDs) sweeps go on until one rotates nothing; with RANGE
+ * rows of any norm are rotated. */
+template <int LP, int G, bool EXACT = false, bool RANGE = false>
 __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int W, int ld, double *red) {
   const int lane = threadIdx.x;
   const double eps = 2.220446049250313e-16;
@@ -434,11 +434,15 @@ __device__ __forceinline__ void jacobi_rows(double2 *__restrict__ M, int p, int 
         be = group_sum(be, LP);
         gx = group_sum(gx, LP);
         gy = group_sum(gy, LP);
-        if (EXACT) pair_range(al, be, gx, gy);
-        const double ag2 = gx * gx + gy * gy;
+        double ag2 = gx * gx + gy * gy;
         /* rows below 1e-145 in norm lie far under any cut; they are not rotated
-         * (without EXACT) */
-        if (valid && ag2 > 1e-290 && ag2 > thr2 * al * be) {
+         * (without RANGE) */
+        bool turn = valid && ag2 > 1e-290 && ag2 > thr2 * al * be;
+        if (RANGE && valid && !turn && pair_range(al, be, gx, gy)) {
+          ag2 = gx * gx + gy * gy;
+          turn = ag2 > thr2 * al * be;
+        }
+        if (turn) {
           rotated = 1;
           big |= ag2 >= 1e-12 * (al * be);
           const double rg = rsqrt_nr(ag2);
@@ -1338,6 +1342,13 @@ __host__ __device__ __forceinline__ int tall_ld(int n) { return 2 * n + 1; }
 /* [R | I] and the reductions of 16 waves */
 __host__ __device__ __forceinline__ size_t svd_tall_lds(int n) { return (size_t)n * tall_ld(n) * 16 + 256; }
 __host__ __device__ __forceinline__ size_t svd_tall_w_lds(int n) { return (size_t)2 * n * n * 16; }
+/* The triangle's first row ends in a flag, in the entry that pads it: whether
+ * products of its rows can leave the range, by the least and the largest
+ * square of a pivot (1e-100 and 1e100: the rows that a sweep leaves may be
+ * smaller than the pivots).  The check of every pair costs the Jacobi 3%. */
+__device__ __forceinline__ double2 tall_range(double least, double most) {
+  return make_double2(least > 1e-100 && most < 1e100 ? 0.0 : 1.0, 0.0);
+}
 /* scratch slot of one matrix of a batch whose widest has maxN columns:
  * [R | I] then [R' | G], n x (2n + 1) */
 static inline int64_t tall_slot(int maxN) { return (int64_t)maxN * (2 * maxN + 1); }
@@ -1376,6 +1387,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
 #pragma unroll
   for (int q = 0; q < CPW; ++q) diag[q] = make_double2(0, 0);
   int rank = n; /* rows of R from here on are zero */
+  double least = 1, most = 1;
   for (int j = 0; j < n; ++j) {
     /* the largest remaining column, the first among equals; where no
      * comparison holds (NaN) the first remaining one */
@@ -1391,6 +1403,8 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
     const int p = __builtin_amdgcn_readfirstlane(bi < n ? bi : free1);
     const double sg = house_norm(cn[p]);
     if (cn[p] <= HOUSE_LEAST) rank = min(rank, j); /* and with it what is left */
+    else least = fmin(least, cn[p]);
+    most = fmax(most, cn[p]);
     if (w == (p & (NW - 1))) { /* the wave that holds it: the reflector */
 #pragma unroll
       for (int q = 0; q < CPW; ++q)
@@ -1466,6 +1480,7 @@ __device__ __forceinline__ void qr_regs(const double2 *__restrict__ a, double2 *
     const int i = e / n, c = e - i * n;
     rg[i * ld + n + c] = make_double2(c == i ? 1.0 : 0.0, 0.0);
   }
+  if (tid == 0) rg[2 * n] = tall_range(least, most);
 }
 
 __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restrict__ idx,
@@ -1514,6 +1529,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
   }
   __syncthreads();
   int rank = n; /* rows of R from here on are zero */
+  double least = 1, most = 1;
   for (int j = 0; j < n; ++j) {
     if (w == 0) { /* the largest remaining column, the first among equals */
       double best = -1.0;
@@ -1546,6 +1562,8 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     double2 *x = s + (int64_t)j * m;
     const double sg = house_norm(qnorm);
     if (qnorm <= HOUSE_LEAST) rank = min(rank, j);
+    else least = fmin(least, qnorm);
+    most = fmax(most, qnorm);
     const double2 x0 = x[j];
     const double ax0 = hypot(x0.x, x0.y);
     const double phx = ax0 > 0 ? x0.x / ax0 : 1.0, phy = ax0 > 0 ? x0.y / ax0 : 0.0;
@@ -1579,6 +1597,7 @@ __global__ __launch_bounds__(SVD_TALL_T) void k_tall_qr(const int32_t *__restric
     else v = make_double2(c - n == i ? 1.0 : 0.0, 0.0);
     rg[i * ld + c] = v;
   }
+  if (tid == 0) rg[2 * n] = tall_range(least, most);
   for (int j = tid; j < n; j += SVD_TALL_T) pivg[(int64_t)t * maxN + j] = pv[j];
 }
 
@@ -1594,11 +1613,14 @@ __global__ __launch_bounds__(T) void k_tall_jacobi(const int32_t *__restrict__ i
   const int npairs = (n + (n & 1)) / 2;
   int Lp = 64;
   while (Lp > 1 && Lp * npairs > T) Lp >>= 1;
-  switch (Lp) {
-    case 64: jacobi_rows<64, T, true>(lds, n, 2 * n, ld, red); break;
-    case 32: jacobi_rows<32, T, true>(lds, n, 2 * n, ld, red); break;
-    default: jacobi_rows<16, T, true>(lds, n, 2 * n, ld, red); break;
-  }
+  if (lds[2 * n].x == 0)
+    switch (Lp) {
+      case 64: jacobi_rows<64, T, true>(lds, n, 2 * n, ld, red); break;
+      case 32: jacobi_rows<32, T, true>(lds, n, 2 * n, ld, red); break;
+      default: jacobi_rows<16, T, true>(lds, n, 2 * n, ld, red); break;
+    }
+  else /* one width of it is enough */
+    jacobi_rows<16, T, true, true>(lds, n, 2 * n, ld, red);
   __syncthreads();
   for (int e = threadIdx.x; e < n * ld; e += T) rg[e] = lds[e];
 }
@@ -1633,6 +1655,7 @@ __global__ __launch_bounds__(SVD_BLK_T) void k_svd_block(const int32_t *__restri
   const int g = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const double eps = 2.220446049250313e-16;
   const double thr = 4.0 * eps * sqrt((double)n), thr2 = thr * thr;
+  const bool range = RG[(int64_t)t * slot + 2 * n].x != 0;
   int rotated = 0;
   const int inner = round == 0 ? SVD_BLK - 1 : 0;
   for (int step = 0; step < inner + SVD_BLK; ++step) {
@@ -1664,9 +1687,13 @@ __global__ __launch_bounds__(SVD_BLK_T) void k_svd_block(const int32_t *__restri
       be = group_sum(be, 64);
       gx = group_sum(gx, 64);
       gy = group_sum(gy, 64);
-      pair_range(al, be, gx, gy);
-      const double ag2 = gx * gx + gy * gy;
-      if (ag2 > 1e-290 && ag2 > thr2 * al * be) { /* the rotation of jacobi_rows */
+      double ag2 = gx * gx + gy * gy;
+      bool turn = ag2 > 1e-290 && ag2 > thr2 * al * be;
+      if (range && !turn && pair_range(al, be, gx, gy)) {
+        ag2 = gx * gx + gy * gy;
+        turn = ag2 > thr2 * al * be;
+      }
+      if (turn) { /* the rotation of jacobi_rows */
         rotated = 1;
         const double rg = rsqrt_nr(ag2);
         const double ex = gx * rg, ey = gy * rg;
