@@ -1065,8 +1065,8 @@ __global__ void k_f32_to_f64(int64_t n, const float2 *__restrict__ a, double2 *_
  * <= 64, so a pair's reduction stays in one wave).  It is left for the
  * matrices of more than 256 rows and less than 2^15 entries.  Through their
  * QR they would take a quarter of the time, with singular values as near (of
- * 300 x 40 to 500 x 60, against long double: 3e-9 to 7e-9 relative at 1e-8 of
- * the largest either way) and U orthonormal to 1e-14 instead of 1e-15; but
+ * 300 x 40 to 500 x 60, against long double at 1e-8 of the largest: 3e-9 to
+ * 5e-9 relative, here 6e-9 to 9e-9) and U orthonormal to 1e-14 (1e-15); but
  * streams of such blocks merge bases known to 1e-8 at a cut of 1e-8, where any
  * rounding decides the rank (406 or 407 columns in all of one stream of 2048
  * points), and the factor shapes they have given stay what they are. */
