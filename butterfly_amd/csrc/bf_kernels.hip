@@ -2228,8 +2228,10 @@ static int g_mfmaCT = -1;
  * 2% in the mixed forms and by -3 to 4% in FP64; the columns split at 4096
  * waves cost the box 8%. */
 /* A wave for each pass of the tallest segment, in every segment (a wave takes
- * every rowGroups-th pass): those that find no pass cost about a nanosecond
- * each, the tallest's chain in fewer waves more. */
+ * every rowGroups-th pass): those that find no pass cost little (4 -> 6 groups
+ * of 9558 segments, 19000 of them, 56.4 -> 57.8 us), the tallest's chain in
+ * fewer waves more (8248 segments, tallest 240 rows, 15 passes in 1 / 4 / 8 / 15
+ * groups 179 / 81 / 69 / 67 us). */
 static int mfma_row_groups(int64_t numSegs, const BfkStageShape &sh, int chunks, int rowTiles) {
   const int64_t n = numSegs * chunks, most = (sh.maxRows + 16 * rowTiles - 1) / (16 * rowTiles);
   if (n >= 16384) return 1;
